@@ -176,7 +176,7 @@ struct mastg_ctx {
     bool mg_k0_set = false;    // problem-level steps chosen by the caller (MASTG_OPT_MG_STEPS_FINE)
     int mg_ratio = 0;          // Chebyshev interval [lam / ratio, lam] (0: the physics' default)
     int64_t mg_n_coarse = 0;   // DOFs of the dense coarsest level
-    DevBuf mg_cheb, mg_lam, mg_part, mg_dense, mg_scal;
+    DevBuf mg_cheb, mg_lam, mg_part, mg_dense, mg_dense_w, mg_scal;
     bool mg_power = false;     // Chebyshev bounds from power iteration (plates)
     hipGraphExec_t mg_exec = nullptr;
     int mg_exec_len = 0;
@@ -931,6 +931,7 @@ int mg_build(mastg_ctx* c) {
     TRY(dalloc(c, c->mg_part, size_t(std::max<int64_t>(8192, (c->S.n_active + 255) / 256 + 1)) * sizeof(double)));
     c->mg_n_coarse = H.coarsest_dofs;
     TRY(dalloc(c, c->mg_dense, size_t(H.coarsest_dofs * H.coarsest_dofs) * sizeof(double)));
+    TRY(dalloc(c, c->mg_dense_w, size_t(mg_invert_work(int(H.coarsest_dofs))) * sizeof(double)));
     TRY(dalloc(c, c->mg_scal, 2 * sizeof(double)));
     // plates: the Gershgorin bound of D^-1 A is loose by ~50x (thin-plate
     // bending against membrane rows); their Chebyshev intervals come from
@@ -1075,9 +1076,10 @@ int mg_setup(mastg_ctx* c) {
     launch_mg_cheb(c->mg_lam.as<double>(), c->mg_cheb.as<double>(), nl, std::max(c->mg_k0, c->mg_kc), ratio, s);
     const MGLevelDev& Lc = *c->mg[nl - 1];
     const int64_t n = c->mg_n_coarse;
-    launch_fill(n * n, 0.0, c->mg_dense.as<double>(), s);
-    launch_mg_dense_gather(Lc.a, c->mg_dense.as<double>(), s);
-    launch_mg_invert(int(n), c->mg_dense.as<double>(), s);
+    double* dense = mg_invert_input(int(n), c->mg_dense.as<double>(), c->mg_dense_w.as<double>());
+    launch_fill(n * n, 0.0, dense, s);
+    launch_mg_dense_gather(Lc.a, dense, s);
+    launch_mg_invert(int(n), c->mg_dense.as<double>(), c->mg_dense_w.as<double>(), s);
     HIPC(c, hipGetLastError());
     c->mg_valid = true;
     return MASTG_OK;

@@ -340,7 +340,12 @@ void launch_mg_galerkin_class(const MGGalerkinArgs& g, hipStream_t s);
 // max_i sum_j |a_ij| / a_ii into *lam; level 0 reads the scalar CSR
 void launch_mg_cheb(const double* lam, double* cheb, int n_levels, int k, double ratio, hipStream_t s);
 void launch_mg_dense_gather(const MGLevelArgs& L, double* A, hipStream_t s);
-void launch_mg_invert(int n, double* A, hipStream_t s);
+// A = the inverse of the n x n matrix in mg_invert_input(n, A, W), one of the
+// two buffers (every block step goes from one to the other); W holds
+// mg_invert_work(n) doubles
+int64_t mg_invert_work(int n);
+double* mg_invert_input(int n, double* A, double* W);
+void launch_mg_invert(int n, double* A, double* W, hipStream_t s);
 // V-cycle pieces; every kernel returns at once when *done != 0 (done may be null)
 void launch_mg_pre_init(const MGLevelArgs& L, const int* done, hipStream_t s);
 // the FP16 row-scaled copy of a lattice-order 27-point stencil ([27][n])

@@ -1042,73 +1042,6 @@ __global__ __launch_bounds__(256) void k_mg_power_start_norm(const double* __res
     if (threadIdx.x == 0) scal[1] = sqrt(s);
 }
 
-// Gauss-Jordan inverse of an SPD matrix (no pivoting), n <= 136, one block of
-// 1024 threads.  Thread t keeps the 9 x 3 entries at rows (t >> 6) + 16 r and
-// columns (t & 63) + 64 c in registers (a 144 x 192 cover of the matrix; the
-// entries outside n x n stay 0).  Pivot k's row lives in wave k & 15 (register
-// row k >> 4) and its column in lane k & 63 of every wave (register column
-// k >> 6), so the owners are known without searching: lane k & 63 publishes
-// the column, the pivot row's wave broadcasts the pivot across its lanes,
-// scales the row in registers and publishes it (entry k = 1 / pivot), and
-// every thread updates its entries with selects instead of branches.  The
-// pivot column and row are double-buffered in LDS, so one barrier per pivot
-// suffices: a buffer is rewritten two pivots later, after every thread has
-// passed the barrier that follows its last read.
-__global__ __launch_bounds__(1024) void k_mg_invert_lds(int n, double* __restrict__ A) {
-    __shared__ double colk[2][144], rowk[2][192];
-    const int t = threadIdx.x, i0 = t >> 6, j0 = t & 63;
-    double a[9][3];
-#pragma unroll
-    for (int r = 0; r < 9; r++)
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-            const int i = i0 + 16 * r, j = j0 + 64 * c;
-            a[r][c] = (i < n && j < n) ? A[i * n + j] : 0.0;
-        }
-    for (int k = 0; k < n; k++) {
-        const int b = k & 1, kr = k >> 4, ki = k & 15, kc = k >> 6, kj = k & 63;
-        if (j0 == kj)   // column k (before this pivot's update)
-#pragma unroll
-            for (int r = 0; r < 9; r++) colk[b][i0 + 16 * r] = kc == 0 ? a[r][0] : (kc == 1 ? a[r][1] : a[r][2]);
-        if (i0 == ki) {   // the pivot row's wave (uniform branch)
-            double rv[3] = {0.0, 0.0, 0.0};
-#pragma unroll
-            for (int r = 0; r < 9; r++)
-#pragma unroll
-                for (int c = 0; c < 3; c++) rv[c] = r == kr ? a[r][c] : rv[c];
-            const double piv = __shfl(kc == 0 ? rv[0] : (kc == 1 ? rv[1] : rv[2]), kj);
-            const double p = 1.0 / piv;
-#pragma unroll
-            for (int c = 0; c < 3; c++) {
-                const int j = j0 + 64 * c;
-                rowk[b][j] = j == k ? p : rv[c] * p;
-            }
-        }
-        __syncthreads();
-        const double p = rowk[b][k];
-        double ck[9], rk[3];
-#pragma unroll
-        for (int r = 0; r < 9; r++) ck[r] = colk[b][i0 + 16 * r];
-#pragma unroll
-        for (int c = 0; c < 3; c++) rk[c] = rowk[b][j0 + 64 * c];
-#pragma unroll
-        for (int r = 0; r < 9; r++)
-#pragma unroll
-            for (int c = 0; c < 3; c++) {
-                const bool is_row = i0 == ki && r == kr, is_col = j0 + 64 * c == k;
-                const double v = is_col ? -ck[r] * p : fma(-ck[r], rk[c], a[r][c]);
-                a[r][c] = is_row ? rk[c] : v;
-            }
-    }
-#pragma unroll
-    for (int r = 0; r < 9; r++)
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-            const int i = i0 + 16 * r, j = j0 + 64 * c;
-            if (i < n && j < n) A[i * n + j] = a[r][c];
-        }
-}
-
 // ---- transfers ---------------------------------------------------------------
 // r_C = sum over the 3^DIM fine points around 2C of w * res_f (w = prod of 1 or
 // 1/2), constrained fine DOFs weighted 0, constrained coarse DOFs zero (P^T),
@@ -1226,23 +1159,134 @@ __global__ __launch_bounds__(256) void k_mg_dense_gather(MGLevelArgs L, double* 
     }
 }
 
-// in-place Gauss-Jordan inverse of an SPD matrix (no pivoting), one block
-__global__ __launch_bounds__(1024) void k_mg_invert(int n, double* __restrict__ A) {
-    __shared__ double colk[1536];
-    for (int k = 0; k < n; k++) {
-        for (int i = threadIdx.x; i < n; i += 1024) colk[i] = A[int64_t(i) * n + k];
-        __syncthreads();
-        const double p = 1.0 / colk[k];
-        for (int j = threadIdx.x; j < n; j += 1024)
-            A[int64_t(k) * n + j] = (j == k) ? p : A[int64_t(k) * n + j] * p;
-        __syncthreads();
-        const int64_t nn = int64_t(n) * n;
-        for (int64_t idx = threadIdx.x; idx < nn; idx += 1024) {
-            const int64_t i = idx / n, j = idx - i * n;
-            if (i == k) continue;
-            A[idx] = (j == k) ? -colk[i] * p : A[idx] - colk[i] * A[int64_t(k) * n + j];
+// Blocked Gauss-Jordan inverse (no pivoting: the coarsest operators are SPD,
+// or the heat Jacobian's, whose symmetric part is), one launch per 32 x 32
+// diagonal block, out of place: with D the kb-th diagonal block of `in`,
+//   out[kb][kb] = D^-1,  out[kb][j] = D^-1 in[kb][j],  out[i][kb] = -in[i][kb] D^-1,
+//   out[i][j] = in[i][j] - in[i][kb] (D^-1 in[kb][j]).
+// Bound by the chain of n pivots, each waiting for the one before it.  A
+// work-group per 32 x 32 tile; the one that updates the next diagonal block
+// also inverts it (Dinv of the next launch), so the pivots run once and not in
+// every work-group (which took 42 us per step at n = 1188, all of them
+// competing for the FP64 units).  Against the whole matrix updated pivot by
+// pivot from one work-group: n = 1188 732 ms -> 0.97 ms, n = 135 (in
+// registers, 1024 threads) 0.25 ms -> 0.10 ms.
+constexpr int kInvB = 32;
+
+// D^-1 of the 32 x 32 block whose entries (r0 + 8 q, c) thread t holds in a,
+// in place: one barrier per pivot, the pivot row and column double-buffered
+// (0.4 us per pivot; every thread dividing for itself instead of the shuffle
+// and scaled row measured 5% slower)
+__device__ __forceinline__ void mg_invert_block(double a[4], double (&colk)[2][kInvB], double (&rowk)[2][kInvB]) {
+    const int t = threadIdx.x, lane = t & 63, c = t & 31, r0 = t >> 5;
+    for (int k = 0; k < kInvB; k++) {
+        const int b = k & 1, kq = k >> 3;
+        if (c == k)
+#pragma unroll
+            for (int q = 0; q < 4; q++) colk[b][r0 + 8 * q] = a[q];
+        if (r0 == (k & 7)) {   // the half wave holding pivot row k
+            const double v = kq == 0 ? a[0] : kq == 1 ? a[1] : kq == 2 ? a[2] : a[3];
+            const double p = 1.0 / __shfl(v, (lane & 32) | k, 64);
+            rowk[b][c] = c == k ? p : v * p;
         }
-        __syncthreads();
+        __syncthreads();   // (a buffer is rewritten two pivots later, past the next barrier)
+        const double p = rowk[b][k], rk = rowk[b][c];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const double ck = colk[b][r0 + 8 * q];
+            const double v = c == k ? -ck * p : fma(-ck, rk, a[q]);
+            a[q] = r0 + 8 * q == k ? rk : v;
+        }
+    }
+}
+
+// entry (row, col) of the matrix; past n the identity's, so a last partial
+// block inverts like a whole one
+__device__ __forceinline__ double mg_invert_load(const double* __restrict__ A, int n, int row, int col) {
+    return row < n && col < n ? A[int64_t(row) * n + col] : (row == col ? 1.0 : 0.0);
+}
+
+// the first diagonal block's inverse
+__global__ __launch_bounds__(256) void k_mg_invert_first(int n, const double* __restrict__ in,
+                                                         double* __restrict__ Dinv) {
+    __shared__ double colk[2][kInvB], rowk[2][kInvB];
+    const int c = threadIdx.x & 31, r0 = threadIdx.x >> 5;
+    double a[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) a[q] = mg_invert_load(in, n, r0 + 8 * q, c);
+    mg_invert_block(a, colk, rowk);
+#pragma unroll
+    for (int q = 0; q < 4; q++) Dinv[(r0 + 8 * q) * kInvB + c] = a[q];
+}
+
+__global__ __launch_bounds__(256) void k_mg_invert_step(int n, int kb, const double* __restrict__ in,
+                                                        double* __restrict__ out, const double* __restrict__ Dinv,
+                                                        double* __restrict__ Dnext) {
+    __shared__ double D[kInvB][kInvB + 1], R[kInvB][kInvB + 1], Cl[kInvB][kInvB + 1];
+    __shared__ double colk[2][kInvB], rowk[2][kInvB];
+    const int c = threadIdx.x & 31, r0 = threadIdx.x >> 5;   // entries (r0 + 8 q, c), q < 4
+    // the tile, tiles counted from the next diagonal block on: the work-group
+    // with the longest way is dealt out first
+    const int nt = gridDim.x;
+    int ib = blockIdx.y + kb + 1, jb = blockIdx.x + kb + 1;
+    ib -= ib >= nt ? nt : 0;
+    jb -= jb >= nt ? nt : 0;
+    const int gi = ib * kInvB, gj = jb * kInvB, gk = kb * kInvB;
+    double o[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const int r = r0 + 8 * q;
+        D[r][c] = Dinv[r * kInvB + c];
+        o[q] = ib != kb && jb != kb ? mg_invert_load(in, n, gi + r, gj + c) : 0.0;
+        if (jb != kb) R[r][c] = mg_invert_load(in, n, gk + r, gj + c);
+        if (ib != kb) Cl[r][c] = mg_invert_load(in, n, gi + r, gk + c);
+    }
+    __syncthreads();
+    if (jb == kb) {
+        if (ib == kb) {
+#pragma unroll
+            for (int q = 0; q < 4; q++) o[q] = D[r0 + 8 * q][c];
+        } else {
+#pragma unroll 8
+            for (int k = 0; k < kInvB; k++) {
+                const double d = D[k][c];
+#pragma unroll
+                for (int q = 0; q < 4; q++) o[q] = fma(-Cl[r0 + 8 * q][k], d, o[q]);
+            }
+        }
+    } else {
+        double x[4] = {0.0, 0.0, 0.0, 0.0};   // D^-1 in[kb][jb]
+#pragma unroll 8
+        for (int k = 0; k < kInvB; k++) {
+            const double v = R[k][c];
+#pragma unroll
+            for (int q = 0; q < 4; q++) x[q] = fma(D[r0 + 8 * q][k], v, x[q]);
+        }
+        if (ib == kb) {
+#pragma unroll
+            for (int q = 0; q < 4; q++) o[q] = x[q];
+        } else {
+            __syncthreads();   // R is read
+#pragma unroll
+            for (int q = 0; q < 4; q++) R[r0 + 8 * q][c] = x[q];
+            __syncthreads();
+#pragma unroll 8
+            for (int k = 0; k < kInvB; k++) {
+                const double v = R[k][c];
+#pragma unroll
+                for (int q = 0; q < 4; q++) o[q] = fma(-Cl[r0 + 8 * q][k], v, o[q]);
+            }
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const int r = gi + r0 + 8 * q;
+        if (r < n && gj + c < n) out[int64_t(r) * n + gj + c] = o[q];
+    }
+    if (ib == kb + 1 && jb == kb + 1) {   // (no such tile in the last step)
+        mg_invert_block(o, colk, rowk);
+#pragma unroll
+        for (int q = 0; q < 4; q++) Dnext[(r0 + 8 * q) * kInvB + c] = o[q];
     }
 }
 
@@ -1432,11 +1476,18 @@ void launch_mg_dense_gather(const MGLevelArgs& L, double* A, hipStream_t s) {
     else
         hipLaunchKernelGGL(k_mg_dense_gather<3>, dim3(mg_blocks(L.n_nodes * 3, 256)), dim3(256), 0, s, L, A);
 }
-void launch_mg_invert(int n, double* A, hipStream_t s) {
-    if (n <= 136)
-        hipLaunchKernelGGL(k_mg_invert_lds, dim3(1), dim3(1024), 0, s, n, A);
-    else
-        hipLaunchKernelGGL(k_mg_invert, dim3(1), dim3(1024), 0, s, n, A);
+int64_t mg_invert_work(int n) { return int64_t(n) * n + 2 * kInvB * kInvB; }
+double* mg_invert_input(int n, double* A, double* W) { return ((n + kInvB - 1) / kInvB) & 1 ? W : A; }
+void launch_mg_invert(int n, double* A, double* W, hipStream_t s) {
+    const int nt = (n + kInvB - 1) / kInvB;
+    double *in = mg_invert_input(n, A, W), *out = in == A ? W : A;   // the last step writes A
+    double *d0 = W + int64_t(n) * n, *d1 = d0 + kInvB * kInvB;
+    hipLaunchKernelGGL(k_mg_invert_first, dim3(1), dim3(256), 0, s, n, in, d0);
+    for (int k = 0; k < nt; k++) {
+        hipLaunchKernelGGL(k_mg_invert_step, dim3(nt, nt), dim3(256), 0, s, n, k, in, out, d0, d1);
+        std::swap(in, out);
+        std::swap(d0, d1);
+    }
 }
 static inline int nb_grid(int64_t n_nodes) {
     const int64_t blocks = (n_nodes * 8 + 255) / 256;

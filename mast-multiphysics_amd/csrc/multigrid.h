@@ -41,7 +41,7 @@ struct MGHierarchy {
 // Largest coarsest-level system solved by the dense inverse.
 constexpr int64_t kMGMaxCoarseDofs = 1536;
 // Coarsening continues while a level has more DOFs than this (and its cell
-// counts are even): the coarsest inverse then fits in LDS.
+// counts are even).
 constexpr int64_t kMGCoarseTarget = 136;
 
 // Detects the lattice and builds the coarse levels (hex8: nav 3, quad4: nav 5).

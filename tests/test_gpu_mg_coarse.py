@@ -1,0 +1,56 @@
+"""The multigrid hierarchy's coarsest level: its blocked dense inverse at the
+edges of its 32 x 32 blocks (whole and partial last blocks, the smallest and
+the largest coarsest systems), through design evaluations at the bars every
+solver meets (compliance 1e-9, gradient 1e-7 of the oracle's).  An inexact
+coarse solve would show as iterations: the bound is twice the V-cycle's usual
+count on these meshes."""
+import pytest
+
+from helpers import ctx_from_oracle, rel_err_floor
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("mesh", [
+    (6, 2, 2),       # 48 coarsest DOFs: one whole block and a half
+    (12, 4, 4),      # the same below one more level
+    (6, 6, 2),       # 96: whole blocks only
+    (10, 10, 10),    # 648
+    (14, 14, 14),    # 1536: the largest
+])
+def test_coarsest_inverse_hex8(oracle, mastg, mesh):
+    print(f"[coarsest inverse] hex8 {mesh}", flush=True)
+    P = oracle.Problem(oracle.CANTILEVER, *mesh, seed=2, lo=0.1, hi=1.0)
+    ref = P.solve_elastic(1e-10)
+    ctx = ctx_from_oracle(mastg, P)
+    r = ctx.design_eval(P.params(), solver=mastg.SOLVER_MG)
+    assert r["rel_res"] <= 1.5e-10 and r["iters"] <= 40, r["iters"]
+    assert abs(r["objective"] - ref["compliance"]) <= 1e-9 * abs(ref["compliance"])
+    assert rel_err_floor(r["grad"], ref["dc"], floor=1e-6) <= 1e-7
+    ctx.close()
+
+
+@pytest.mark.parametrize("n", [6, 10])   # 64 (two whole blocks) and 216 coarsest DOFs, not symmetric
+def test_coarsest_inverse_heat(oracle, mastg, n):
+    print(f"[coarsest inverse] heat {n}^3", flush=True)
+    P = oracle.Problem(oracle.HEAT, n, seed=5)
+    ref = P.solve_heat(1e-12, 1e-14)
+    ctx = ctx_from_oracle(mastg, P)
+    r = ctx.design_eval(P.params(), rtol=1e-12, solver=mastg.SOLVER_MG)
+    assert r["iters"] <= 12 * (r["newton_iters"] + 1), (r["iters"], r["newton_iters"])
+    assert abs(r["objective"] - ref["mean_T"]) <= 1e-9 * abs(ref["mean_T"])
+    assert rel_err_floor(r["grad"], ref["dJ"], floor=1e-6) <= 1e-7
+    ctx.close()
+
+
+def test_coarsest_inverse_plate(oracle, mastg):
+    """10 x 10 cells: 180 coarsest DOFs."""
+    print("[coarsest inverse] plate 10x10", flush=True)
+    P = oracle.Problem(oracle.PLATE, 10, 10, seed=1)
+    ref = P.solve_elastic(1e-10)
+    ctx = ctx_from_oracle(mastg, P)
+    r = ctx.design_eval(P.params(), solver=mastg.SOLVER_MG)
+    assert r["rel_res"] <= 1.5e-10 and r["iters"] * 4 < ref["iters"], (r["iters"], ref["iters"])
+    assert abs(r["objective"] - ref["compliance"]) <= 1e-9 * abs(ref["compliance"])
+    assert rel_err_floor(r["grad"], ref["dc"], floor=1e-6) <= 1e-7
+    ctx.close()
