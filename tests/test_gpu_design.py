@@ -56,6 +56,34 @@ def test_filter_and_volume(oracle, mastg, kind, mesh, r_h, distort):
     Dg.close()
 
 
+# rows by pattern: every row its own pattern (4 x 4 x 4, the ball covers the
+# mesh), one element, waves of 64 rows cut by every boundary, a pattern of
+# exactly one batch of 16 and of 17; and more distinct rows than patterns are
+# kept for (displaced nodes: the CSR)
+@pytest.mark.parametrize("mesh,r_h,distort", [((4, 4, 4), 9.0, 0.0), ((1, 1, 1), 1.5, 0.0), ((65, 2, 3), 1.5, 0.0),
+                                              ((64, 4, 4), 1.2, 0.0), ((16, 1, 1), 20.0, 0.0), ((17, 1, 1), 20.0, 0.0),
+                                              ((20, 16, 16), 1.8, 0.2)])
+def test_filter_row_patterns(oracle, mastg, mesh, r_h, distort):
+    print(f"[filter row patterns] {mesh} r = {r_h} h, distortion {distort}", flush=True)
+    P = oracle.Problem(oracle.CANTILEVER, *mesh, seed=2, lo=0.3, hi=1.0)
+    _, xyz, conn = _desc(mastg, P)
+    h = 1.0 / mesh[0]
+    xyz = xyz + distort * h * np.random.default_rng(4).uniform(-0.5, 0.5, xyz.shape)
+    r = r_h * h * 1.0000001          # no neighbour at exactly the radius
+    Dg = mastg.Design(mastg.desc_from_arrays(mastg.HEX8_ELASTIC, xyz, conn, P.n_vars), r)
+    c = D.centroids(xyz, conn)
+    W = D.filter_matrix(c, r)
+    x = np.random.default_rng(1).uniform(0.0, 1.0, P.n_elems)
+    # a weight r - d carries the rounding of the coordinates' differences (16
+    # eps of the largest coordinate at most, the bound rows are matched to) on
+    # either side
+    tol = 1e-14 + 32 * 2.2e-16 * np.abs(c).max() / r
+    for t, M in ((False, W), (True, W.T)):
+        y = M @ x
+        assert np.max(np.abs(Dg.filter(x, transpose=t) - y)) <= tol * np.abs(y).max()
+    Dg.close()
+
+
 def test_oc_update(oracle, mastg):
     print("[design OC] hex8 16x8x8", flush=True)
     P = oracle.Problem(oracle.CANTILEVER, 16, 8, 8, seed=2, lo=0.3, hi=1.0)
