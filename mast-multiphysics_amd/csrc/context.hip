@@ -99,7 +99,8 @@ struct MGLevelDev {
     MGLevelArgs a{};
     int64_t n_elems = 0;
     DevBuf rank_of_lat, elem_of_cell, con_lat, nodecon_lat, dinv_lat, b_lat, sE_cell;   // level 0
-    DevBuf x32, res32, da32, db32, dinv32, y_lat;   // hex8 level 0: FP32 smoothing state, FP64 scratch
+    DevBuf x32, y32, b32, res32, dinv32, y_lat;   // hex8 level 0: FP32 smoothing state, FP64 scratch
+    DevBuf sE_cell32;                             // FP32 copy of sE_cell
     DevBuf blk_ptr, blk_col, cptr, cidx, econn, con;   // levels >= 1
     DevBuf gal_dirty, gal_list;   // hex8 level 1: coarse cells touching constraints
     int64_t n_dirty = 0;
@@ -130,6 +131,9 @@ struct mastg_ctx {
     DevBuf Khat, sE, eclass, nodecon, Fel;
     DevBuf heat_geo;            // heat: per congruence class gradients and JxW
     DevBuf Khat32;              // FP32 copy of Khat (lattice smoothing)
+    bool is_box = false;        // Khat is an axis-aligned box's: box, box32
+    BoxOp<double> box{};
+    BoxOp<float> box32{};
     DevBuf Gc;                  // [8][576] Q_c^T Khat Q_c (lattice Galerkin products)
     // heat: convective side masks, mean-T weights, BiCGStab work space, A^T values
     DevBuf sidemask, radmask, wmean, tpos, valT, vr0, vv, vs, vt, vph, vsh, bscal, vT;
@@ -707,8 +711,8 @@ void ensure_scales(mastg_ctx* c) {
     }
     if (!c->sEc_valid && !c->mg.empty() && !c->mg_power) {
         const MGLevelDev& L0 = *c->mg[0];
-        launch_gather_values(L0.n_elems, L0.elem_of_cell.as<int32_t>(), c->sE.as<double>(),
-                             const_cast<double*>(L0.sE_cell.as<double>()), c->stream);
+        launch_gather_values2(L0.n_elems, L0.elem_of_cell.as<int32_t>(), c->sE.as<double>(),
+                              L0.sE_cell.as<double>(), L0.sE_cell32.as<float>(), c->stream);
         c->sEc_valid = true;
     }
 }
@@ -851,16 +855,13 @@ int mg_build(mastg_ctx* c) {
             a.planar = 1;
             // FP32 smoothing state; y_lat: FP64 lattice-ordered scratch for
             // operator products outside the solve
-            TRY(dalloc(c, L->x32, nv / 2));
-            TRY(dalloc(c, L->res32, nv / 2));
-            TRY(dalloc(c, L->da32, nv / 2));
-            TRY(dalloc(c, L->db32, nv / 2));
-            TRY(dalloc(c, L->dinv32, nv / 2));
+            for (DevBuf* b : {&L->x32, &L->y32, &L->b32, &L->res32, &L->dinv32}) TRY(dalloc(c, *b, nv / 2));
             TRY(dalloc(c, L->y_lat, nv));
+            TRY(dalloc(c, L->sE_cell32, size_t(h.n_elems) * sizeof(float)));
             a.x32 = L->x32.as<float>();
+            a.y32 = L->y32.as<float>();
+            a.b32 = L->b32.as<float>();
             a.res32 = L->res32.as<float>();
-            a.da32 = L->da32.as<float>();
-            a.db32 = L->db32.as<float>();
             a.dinv32 = L->dinv32.as<float>();
             TRY(dalloc(c, c->Khat32, 64 * 9 * sizeof(float)));
             launch_to_f32(64 * 9, c->Khat.as<double>(), c->Khat32.as<float>(), c->stream);
@@ -915,6 +916,20 @@ int mg_build(mastg_ctx* c) {
             HIPC(c, hipMemcpy(Kh.data(), c->Khat.p, Kh.size() * sizeof(double), hipMemcpyDeviceToHost));
         }
         mg_class_child_products(Kh.data(), G.data());
+        c->is_box = box_operator(Kh.data(), c->box);
+        const double* b64 = &c->box.d[0][0];
+        float* b32 = &c->box32.d[0][0];
+        static_assert(sizeof(BoxOp<double>) == 2 * sizeof(BoxOp<float>), "the same layout");
+        for (size_t i = 0; i < sizeof(c->box) / sizeof(double); i++) b32[i] = float(b64[i]);
+        // partial sums of the lattice kernels' grids
+        LatticeOpArgs lat{};
+        lat.nx = H.levels[0].nx; lat.ny = H.levels[0].ny; lat.nz = H.levels[0].nz;
+        const size_t np = size_t(lattice_partials_most(lat)) * sizeof(double);
+        if (c->part0.bytes < np) {
+            drop_graphs(c);   // captured solvers hold the buffers' addresses
+            TRY(dalloc(c, c->part0, np));
+            TRY(dalloc(c, c->part1, np));
+        }
         TRY(upload(c, c->Gc, G));
         std::vector<uint8_t> dirty;
         std::vector<int32_t> list;
@@ -1096,13 +1111,18 @@ bool lattice_args(mastg_ctx* c, CGArgs& a) {
     a.lat.Khat = c->Khat.as<double>();
     a.lat.Khat32 = c->Khat32.as<float>();
     a.lat.nodecon = L0.nodecon_lat.as<uint8_t>();
-    return lattice_partials(a.lat) <= int64_t(c->part0.bytes / sizeof(double));
+    a.lat.is_box = c->is_box ? 1 : 0;
+    a.lat.sE_cell32 = L0.sE_cell32.as<float>();
+    a.lat.box = c->box;
+    a.lat.box32 = c->box32;
+    return lattice_partials_most(a.lat) <= int64_t(c->part0.bytes / sizeof(double));
 }
 
 // one V-cycle on the problem-level vector r0 (null: the level-0 args' r); the
-// level-0 output is x0 + dlast0 (formed by the caller): the returned dlast0
-// is FP32 on the hex8 problem level (its smoothing state), else FP64
-// (started: the caller has written the problem level's pre-smoothing start)
+// level-0 output is x0 + dlast0 (formed by the caller): returns dlast0.  The
+// matrix-free hex8 problem level (FP32) returns the output itself, with the
+// partial sums of r . output in a.part0 (started: the caller has written its
+// pre-smoothing start; the convergence test then runs beside the first pass)
 const void* mg_vcycle(mastg_ctx* c, const CGArgs& a, const int* done, hipStream_t s, const double* r0 = nullptr,
                       bool started = false) {
     const int nl = int(c->mg.size());
@@ -1122,13 +1142,26 @@ const void* mg_vcycle(mastg_ctx* c, const CGArgs& a, const int* done, hipStream_
     }
     auto lv = [&](int l) -> const MGLevelArgs& { return l == 0 ? L0 : c->mg[l]->a; };
     auto dbuf = [&](int l, int i) { return (i % 2 == 0) ? lv(l).da : lv(l).db; };
-    auto dbuf32 = [&](int i) { return (i % 2 == 0) ? L0.da32 : L0.db32; };
+    // FP32 problem level: the current iterate in L0.x32, the other in L0.y32
+    LatSmooth S0{};
+    auto fine = [&](int step, bool first, bool resid, bool last) {
+        S0.x = L0.x32;
+        S0.xp = first ? nullptr : L0.y32;
+        S0.b = L0.b32;
+        S0.dinv = L0.dinv32;
+        S0.out = resid ? nullptr : L0.y32;
+        S0.res = resid ? L0.res32 : nullptr;
+        S0.cheb = L0.cheb;
+        S0.step = step;
+        S0.r = last ? L0.r : nullptr;
+        S0.part = last ? a.part0 : nullptr;
+        launch_lattice_smooth(a.lat, S0, done, s);
+        S0.check = CGCheck{};
+        if (!resid) std::swap(L0.x32, L0.y32);
+    };
     // smoothing step from direction buffer iin to iout (-1: none)
     auto apply = [&](int l, int mode, int step, int iin, int iout) {
-        if (l == 0 && f32)
-            launch_mg_fine(a, L0, mode, step, iin < 0 ? nullptr : dbuf32(iin), iout < 0 ? nullptr : dbuf32(iout),
-                           done, s);
-        else if (l == 0 && D0.lat0 && L0.nav == 3)
+        if (l == 0 && D0.lat0 && L0.nav == 3)
             launch_mg_stencil(L0, D0.sten.as<float>(), mode, step, iin < 0 ? nullptr : dbuf(l, iin),
                               iout < 0 ? nullptr : dbuf(l, iout), done, s);
         else if (l == 0 && D0.lat0)
@@ -1149,8 +1182,14 @@ const void* mg_vcycle(mastg_ctx* c, const CGArgs& a, const int* done, hipStream_
         const int k = steps(l);
         // coarse levels start their pre-smoothing inside the restriction
         if (l == 0 && !started) launch_mg_pre_init(lv(l), done, s);
-        for (int i = 1; i < k; i++) apply(l, MG_STEP, i, i - 1, i);
-        apply(l, MG_FINAL, 0, k - 1, -1);
+        if (l == 0 && f32) {
+            if (started) S0.check = CGCheck{a.S, a.part1, a.nvec};
+            for (int i = 1; i < k; i++) fine(i, i == 1, false, false);
+            fine(0, true, true, false);
+        } else {
+            for (int i = 1; i < k; i++) apply(l, MG_STEP, i, i - 1, i);
+            apply(l, MG_FINAL, 0, k - 1, -1);
+        }
         launch_mg_restrict(lv(l), lv(l + 1), done, s);
     }
     const MGLevelArgs& Lc = lv(nl - 1);
@@ -1159,21 +1198,22 @@ const void* mg_vcycle(mastg_ctx* c, const CGArgs& a, const int* done, hipStream_
     for (int l = nl - 2; l >= 0; l--) {
         const int k = steps(l);
         launch_mg_prolong(lv(l), lv(l + 1), dlast, done, s);
+        if (l == 0 && f32) {
+            for (int i = 0; i < k; i++) fine(i, i == 0, false, i == k - 1);
+            return L0.x32;
+        }
         apply(l, MG_RESID_INIT, 0, -1, 0);
         for (int i = 1; i < k; i++) apply(l, MG_STEP, i, i - 1, i);
         if (l > 0) dlast = dbuf(l, k - 1);
     }
-    const int k0 = steps(0);
-    return f32 ? static_cast<const void*>(dbuf32(k0 - 1)) : static_cast<const void*>(dbuf(0, k0 - 1));
+    return dbuf(0, steps(0) - 1);
 }
 
 // z = x0 + dlast0 on the problem level and the partial sums of r.z
 void mg_rz(mastg_ctx* c, const CGArgs& a, const void* dl, hipStream_t s) {
     const MGLevelDev& D0 = *c->mg[0];
     const MGLevelArgs& L0 = D0.a;
-    if (L0.planar) {
-        launch_pcg_rz32(a, L0.x32, static_cast<const float*>(dl), s);
-    } else if (D0.lat0) {   // z = x0 + dlast back in rank order, then r.z
+    if (D0.lat0) {   // z = x0 + dlast back in rank order, then r.z
         launch_mg_combine_rank(L0.n_nodes, L0.nav, L0.rank_of_lat, L0.x, static_cast<const double*>(dl), a.z,
                                &a.S->done, s);
         launch_pcg_rz(a, a.z, nullptr, s);
@@ -1184,13 +1224,32 @@ void mg_rz(mastg_ctx* c, const CGArgs& a, const void* dl, hipStream_t s) {
 
 void mg_pcg_iteration(mastg_ctx* c, const CGArgs& a, hipStream_t s) {
     const int* done = &a.S->done;
-    launch_cg_op_alpha(a, s);
     const MGLevelArgs& L0 = c->mg[0]->a;
-    if (L0.planar) launch_pcg_update_mg(a, L0, s);   // also starts the level-0 smoothing
-    else launch_pcg_update(a, s);
-    mg_rz(c, a, mg_vcycle(c, a, done, s, nullptr, L0.planar != 0), s);
+    if (L0.planar) {   // the lattice solver: no kernel for scalars alone
+        launch_lattice_apply(a, a.p, a.q, s);
+        launch_pcg_update_lat(a, L0, s);   // also starts the level-0 smoothing
+        const void* z = mg_vcycle(c, a, done, s, nullptr, true);
+        launch_pcg_p_lat(a, static_cast<const float*>(z), int(lattice_partials(a.lat)), 0, s);
+        return;
+    }
+    launch_cg_op_alpha(a, s);
+    launch_pcg_update(a, s);
+    mg_rz(c, a, mg_vcycle(c, a, done, s), s);
     launch_pcg_beta(a, s);
     launch_cg_p(a, s);
+}
+
+// z = M r and p = z, from the residual in a.r (the start of PCG, and its restarts)
+int mg_pcg_begin(mastg_ctx* c, const CGArgs& a, hipStream_t s) {
+    const void* z = mg_vcycle(c, a, &a.S->done, s);
+    if (c->mg[0]->a.planar) {
+        launch_pcg_p_lat(a, static_cast<const float*>(z), int(lattice_partials(a.lat)), 1, s);
+        return MASTG_OK;
+    }
+    mg_rz(c, a, z, s);
+    launch_pcg_start2(a, s);
+    HIPC(c, hipMemcpyAsync(a.p, a.z, c->S.n_active * sizeof(double), hipMemcpyDeviceToDevice, s));
+    return MASTG_OK;
 }
 
 int mg_solve(mastg_ctx* c, const double* b, const mastg_solve_opts* o, mastg_solve_stats* st) {
@@ -1227,9 +1286,7 @@ int mg_solve(mastg_ctx* c, const double* b, const mastg_solve_opts* o, mastg_sol
     launch_fill(S.n_active, 0.0, a.x, c->stream);
     HIPC(c, hipMemcpyAsync(a.r, bl, S.n_active * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
     launch_pcg_start(a, bl, rtol * rtol, max_it, c->stream);
-    mg_rz(c, a, mg_vcycle(c, a, &a.S->done, c->stream), c->stream);
-    launch_pcg_start2(a, c->stream);
-    HIPC(c, hipMemcpyAsync(a.p, a.z, S.n_active * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
+    TRY(mg_pcg_begin(c, a, c->stream));
     HIPC(c, hipMemcpyAsync(c->h_scal, a.S, sizeof(CGScalars), hipMemcpyDeviceToHost, c->stream));
     HIPC(c, hipStreamSynchronize(c->stream));
     int done = c->h_scal->done;
@@ -1267,9 +1324,7 @@ int mg_solve(mastg_ctx* c, const double* b, const mastg_solve_opts* o, mastg_sol
                 if (rr < 0.25 * best2) stalls = 0;
                 else if (++stalls >= 8) { done = 5; break; }
                 best2 = std::min(best2, rr);
-                mg_rz(c, a, mg_vcycle(c, a, &a.S->done, c->stream), c->stream);
-                launch_pcg_start2(a, c->stream);
-                HIPC(c, hipMemcpyAsync(a.p, a.z, S.n_active * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
+                TRY(mg_pcg_begin(c, a, c->stream));
             }
         }
     }
@@ -2637,7 +2692,10 @@ int mastg_bench_kernel(mastg_ctx* c, int kind, int n_launch, double* avg_ms) {
             case 10: (void)assemble_active(c, c->vx.as<double>(), true, true); break;
             case 8: {
                 const MGLevelArgs& L0 = c->mg[0]->a;
-                launch_mg_fine(a, L0, MG_STEP, 1, L0.da32, L0.db32, nullptr, c->stream);
+                LatSmooth S{};
+                S.x = L0.x32; S.xp = L0.y32; S.out = L0.y32;
+                S.b = L0.b32; S.dinv = L0.dinv32; S.cheb = L0.cheb; S.step = 1;
+                launch_lattice_smooth(a.lat, S, nullptr, c->stream);
                 break;
             }
             default: break;
@@ -2664,7 +2722,7 @@ int mastg_bench_kernel(mastg_ctx* c, int kind, int n_launch, double* avg_ms) {
         ensure_scales(c);
         TRY(mg_setup(c));
         const MGLevelDev& L0 = *c->mg[0];
-        for (const DevBuf* b : {&L0.x32, &L0.res32, &L0.da32, &L0.db32})
+        for (const DevBuf* b : {&L0.x32, &L0.y32, &L0.b32, &L0.res32})
             HIPC(c, hipMemsetAsync(b->p, 0, b->bytes, c->stream));
     }
     if (kind == 7) {

@@ -2,6 +2,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include "kernels.h"
+
 namespace mastg {
 
 // XCD-aware work-group order.  The dispatcher deals work-groups to the 8 XCDs
@@ -55,6 +57,40 @@ __device__ __forceinline__ void block_max_store(double v, double* partials, int 
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
     if (threadIdx.x == 0) partials[slot] = fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
+}
+
+// one work-group of 256: ||r||^2 of the updated residual, the iteration count
+// and convergence
+__device__ __forceinline__ void pcg_check_block(const CGCheck& C) {
+    const double rr = reduce_partials(C.part, C.n);
+    if (threadIdx.x == 0) {
+        CGScalars* S = C.S;
+        S->rr = rr;
+        S->iter += 1;
+        if (!isfinite(rr)) S->done = 4;
+        else if (rr <= S->tol2 * S->bb) S->done = 1;
+        else if (S->iter >= S->max_it) S->done = 2;
+    }
+}
+
+// the coefficients of a lattice smoothing pass, and its update of one value
+// (y = A x there); returns the value's share of r . out
+struct LatCoef {
+    float c1, c2;
+};
+__device__ __forceinline__ LatCoef lat_coef(const LatSmooth& S) {
+    return S.step > 0 ? LatCoef{float(S.cheb[2 * S.step]), float(S.cheb[2 * S.step + 1])} : LatCoef{0.f, float(S.cheb[0])};
+}
+__device__ __forceinline__ double lat_point(const LatSmooth& S, const LatCoef& c, int64_t i, float y, float x, float b,
+                                            float dinv, float xp) {
+    const float res = b - y;
+    if (S.res) {
+        S.res[i] = res;
+        return 0.0;
+    }
+    const float z = x + (c.c1 * (x - xp) + c.c2 * dinv * res);
+    S.out[i] = z;
+    return S.part ? S.r[i] * double(z) : 0.0;
 }
 
 }  // namespace mastg

@@ -130,6 +130,34 @@ struct ScatterArgs {
 struct CGScalars {
     double rz, pq, rr, bb, alpha, beta, tol2;
     int iter, max_it, done, pad;
+    double rz2[2];   // the lattice solver's r.z of iteration i in rz2[i & 1]
+};
+
+// the convergence test of a CG iteration, done by one work-group beside other
+// work: ||r||^2 from its partial sums (S null: no test)
+struct CGCheck {
+    CGScalars* S;
+    const double* part;
+    int n;
+};
+
+// One pass of the hex8 problem level's FP32 Chebyshev smoothing, as the
+// three-term recurrence
+//   out = x + c1 (x - xp) + c2 dinv (b - A x)
+// (step i > 0: c1, c2 = cheb[2 i], cheb[2 i + 1]; step 0: c1 = 0, c2 =
+// cheb[0]; xp null: 0), which reads the iterate of two passes ago only at its
+// own point, so `out` may be xp: five vectors move per pass (x, xp, b, dinv,
+// out) where the form with a running residual and direction moved seven.  res
+// non-null: res = b - A x instead.  part non-null: the partial sums of r . out
+// (FP64) besides.
+struct LatSmooth {
+    const float *x, *xp, *b, *dinv;
+    float *out, *res;
+    const double* cheb;
+    int step;
+    const double* r;
+    double* part;
+    CGCheck check;
 };
 
 // node-centric matrix-free operator over congruence classes (hex8, nav = 3)
@@ -147,6 +175,19 @@ struct MFArgs {
     double* Fel;              // [24][n_elems] element forces (SoA), phase 1 -> phase 2
 };
 
+// the class matrix of an axis-aligned box in the sum / difference modes of its
+// nodes (bit 0 / 1 / 2 of a mode: difference along x / y / z): what does not
+// vanish.  d[v][m]: mode m of component v on itself; for the axis pairs (x, y),
+// (x, z), (y, z) = (a, b), k the third axis: l0 couples modes {a} of u_a and {b}
+// of u_b, l1 {a, k} and {b, k}, m0 {b} of u_a and {a} of u_b, m1 {b, k} and {a, k}
+template <typename T>
+struct BoxOp {
+    T d[3][8];
+    T l0[3], l1[3], m0[3], m1[3];
+};
+// false when Khat ([64][3 x 3]) has other entries (cells that are no boxes)
+bool box_operator(const double* Khat, BoxOp<double>& op);
+
 // matrix-free hex8 operator on a lattice mesh, evaluated per node with
 // vectors in lattice order: y_n = sum over the (up to 8) cells at n of
 // s_e Khat[a_n][b] x_b, constrained rows as diag = cells at the node (inputs
@@ -158,9 +199,15 @@ struct LatticeOpArgs {
     const double* Khat;                // [64*9] the (single) class matrix at E = 1
     const float* Khat32;               // its FP32 copy (the FP32 smoothing steps)
     const uint8_t* nodecon;            // [lattice points] bit v = variable v constrained
+    int is_box;                        // cells are axis-aligned boxes: box, box32 hold the operator
+    const float* sE_cell32;            // FP32 copy of sE_cell (the FP32 smoothing steps)
+    BoxOp<double> box;
+    BoxOp<float> box32;
 };
-// partial sums the lattice operator writes (its grid)
+// partial sums the lattice operator and its smoothing pass write (their grid),
+// and the most they can
 int64_t lattice_partials(const LatticeOpArgs& l);
+int64_t lattice_partials_most(const LatticeOpArgs& l);
 
 struct CGArgs {
     int64_t n;
@@ -175,7 +222,7 @@ struct CGArgs {
     int nvec;                 // grid of the CG vector kernels (and their partials)
     CGScalars* S;
     int use_mf;               // operator: 0 CSR SpMV, 1 matrix-free, 2 FP32 node-block SpMV,
-                              // 3 hex8 lattice operator, 4 FP64 node-block SpMV
+                              // 3 hex8 lattice operator (PCG only), 4 FP64 node-block SpMV
     int spmv_sw;              // CSR SpMV lanes per row (4, 8, 16, 32, 64)
     MFArgs mf;
     // FP32 copy of the CSR values read by node blocks (operator 2): node rank
@@ -209,6 +256,8 @@ void launch_bicg_iteration(const BiCGArgs& a, hipStream_t s);
 // dinv s | t = A sh, x, r, check) so a preconditioner can replace ph and sh
 void launch_bicg_part(const BiCGArgs& a, int part, hipStream_t s);
 void launch_gather_values(int64_t n, const int32_t* idx, const double* src, double* dst, hipStream_t s);
+// the same into dst and its FP32 copy dst32
+void launch_gather_values2(int64_t n, const int32_t* idx, const double* src, double* dst, float* dst32, hipStream_t s);
 
 void launch_to_f32(int64_t n, const double* src, float* dst, hipStream_t s);
 // dst[0:n) = src[0:n) (n even, 16-byte aligned buffers)
@@ -295,9 +344,9 @@ struct MGLevelArgs {
     const double* dinv;                // [nav n_nodes] inverse diagonal
     double *r, *x, *res, *da, *db;     // right side, iterate, residual, smoothing directions
     const double* cheb;                // this level's Chebyshev coefficients
-    // the hex8 problem level (planar) smooths in FP32: iterate, residual,
-    // directions and inverse diagonal (r stays the FP64 CG residual)
-    float *x32, *res32, *da32, *db32;
+    // the hex8 problem level (planar) smooths in FP32: two iterates, right
+    // side, residual and inverse diagonal (r stays the FP64 CG residual)
+    float *x32, *y32, *b32, *res32;
     const float* dinv32;
     // the plate problem level smooths with block Jacobi: the inverses of its
     // 5 x 5 diagonal node blocks ([n_nodes][25], null: point Jacobi)
@@ -384,13 +433,16 @@ void launch_mg_gather_stencil3(const MGLevelArgs& L, const int32_t* rank_of_lat,
 constexpr int kMGHalfStencil = 123;   // FP32 entries per point of the symmetric half 27-point 3x3 stencil
 void launch_mg_stencil(const MGLevelArgs& L, const float* sten, int mode, int step, const double* din, double* dout,
                        const int* done, hipStream_t s);
-// level 0 (hex8): FP32 smoothing step with the lattice operator (c.lat) and
-// the row-local epilogue on L's FP32 state
-void launch_mg_fine(const CGArgs& c, const MGLevelArgs& L, int mode, int step, const float* din, float* dout,
-                    const int* done, hipStream_t s);
+// level 0 (hex8): one pass of the FP32 smoothing with the lattice operator
+void launch_lattice_smooth(const LatticeOpArgs& l, const LatSmooth& S, const int* done, hipStream_t s);
 // y = A x with the lattice operator (lattice-ordered vectors) and partial sums
 // of x.y into c.part0
 void launch_lattice_apply(const CGArgs& c, const double* x, double* y, hipStream_t s);
+// the same two on a lattice of axis-aligned boxes (l.is_box; lattice_box.hip)
+int64_t box_partials(const LatticeOpArgs& l);
+int64_t box_partials_most(const LatticeOpArgs& l);
+void launch_box_apply(const LatticeOpArgs& l, const double* x, double* y, double* part, const int* done, hipStream_t s);
+void launch_box_smooth(const LatticeOpArgs& l, const LatSmooth& S, const int* done, hipStream_t s);
 // inverse diagonal of the lattice operator (component-major lattice order,
 // FP64 and FP32) and lambda_max(D^-1 A) <= max Gershgorin ratio into *lam, with
 // the assembled entries formed from the class matrix and the cell scales
@@ -414,11 +466,13 @@ void launch_mg_coarse_solve(int n, const double* Ainv, const double* r, double* 
                             hipStream_t s);
 // preconditioned CG around the V-cycle
 void launch_pcg_update(const CGArgs& c, hipStream_t s);
-// the same, also starting the pre-smoothing of the FP32 problem level L (hex8)
-void launch_pcg_update_mg(const CGArgs& c, const MGLevelArgs& L, hipStream_t s);
+// the lattice solver's: alpha = r.z / p.q from the operator's partial sums, the
+// update, and the start of the FP32 problem level L's pre-smoothing; the
+// convergence test follows beside the first smoothing pass (CGCheck)
+void launch_pcg_update_lat(const CGArgs& c, const MGLevelArgs& L, hipStream_t s);
+// its direction: r.z from n partial sums in c.part0, p = z (first) or z + beta p
+void launch_pcg_p_lat(const CGArgs& c, const float* z, int n, int first, hipStream_t s);
 void launch_pcg_rz(const CGArgs& c, const double* x0, const double* dlast, hipStream_t s);
-// the same from the FP32 problem-level state of the hex8 V-cycle
-void launch_pcg_rz32(const CGArgs& c, const float* x0, const float* dlast, hipStream_t s);
 void launch_pcg_start(const CGArgs& c, const double* b, double tol2, int max_it, hipStream_t s);
 void launch_pcg_start2(const CGArgs& c, hipStream_t s);
 // r.r of the current r (a restart's true residual): done = 1 / 0 / 2 as it meets tol

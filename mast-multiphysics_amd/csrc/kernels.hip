@@ -1434,6 +1434,15 @@ __global__ void k_gather_values(int64_t n, const int32_t* __restrict__ idx, cons
     if (i < n) dst[i] = src[idx[i]];
 }
 
+__global__ void k_gather_values2(int64_t n, const int32_t* __restrict__ idx, const double* __restrict__ src,
+                                 double* __restrict__ dst, float* __restrict__ dst32) {
+    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const double v = src[idx[i]];
+    dst[i] = v;
+    dst32[i] = float(v);
+}
+
 // ---------------------------------------------------------- launchers ----
 static inline unsigned blocks_for(int64_t n, int per) { return unsigned((n + per - 1) / per); }
 
@@ -1605,6 +1614,9 @@ void launch_bicg_iteration(const BiCGArgs& a, hipStream_t s) {
 void launch_gather_values(int64_t n, const int32_t* idx, const double* src, double* dst, hipStream_t s) {
     hipLaunchKernelGGL(k_gather_values, dim3(blocks_for(n, 256)), dim3(256), 0, s, n, idx, src, dst);
 }
+void launch_gather_values2(int64_t n, const int32_t* idx, const double* src, double* dst, float* dst32, hipStream_t s) {
+    hipLaunchKernelGGL(k_gather_values2, dim3(blocks_for(n, 256)), dim3(256), 0, s, n, idx, src, dst, dst32);
+}
 void launch_elem_scale(int64_t n, const double* rho, double E0, double penalty, double* sE,
                        hipStream_t s) {
     hipLaunchKernelGGL(k_elem_scale, dim3(blocks_for(n, 256)), dim3(256), 0, s, n, rho, E0, penalty, sE);
@@ -1637,9 +1649,7 @@ void launch_mf_elem(const CGArgs& c, const double* x, hipStream_t s) {
         hipLaunchKernelGGL(k_hex8_mf_elem<false>, dim3(ge), dim3(256), 0, s, c, x);
 }
 void launch_cg_op_alpha(const CGArgs& c, hipStream_t s) {
-    if (c.use_mf == 3)
-        launch_lattice_apply(c, c.p, c.q, s);
-    else if (c.use_mf == 1)
+    if (c.use_mf == 1)
         mf_dispatch(c, c.p, c.p, c.q, 1, s);
     else if (c.use_mf == 2)
         nb32_dispatch(c, c.p, c.q, 1, 1, s);

@@ -271,15 +271,14 @@ __global__ __launch_bounds__(256) void k_mg_block_dinv5(MGLevelArgs L, float* __
         for (int w = 0; w < 5; w++) dinvb[n * 25 + v * 5 + w] = float(a[v][w]);
 }
 
-// the same start on the FP32 state of the hex8 problem level
+// the FP32 start of the hex8 problem level: b = r, x = D^-1 b / theta
 __global__ __launch_bounds__(256) void k_mg_pre_init32(MGLevelArgs L, const int* __restrict__ done) {
     if (done && *done) return;
     const float ith = float(L.cheb[0]);
     for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < L.n_nodes * L.nav; i += int64_t(gridDim.x) * 256) {
         const float r = float(L.r[i]);
-        L.x32[i] = 0.f;
-        L.res32[i] = r;
-        L.da32[i] = L.dinv32[i] * r * ith;
+        L.b32[i] = r;
+        L.x32[i] = L.dinv32[i] * r * ith;
     }
 }
 
@@ -646,6 +645,7 @@ __global__ __launch_bounds__(256) void k_mg_combine_rank(int64_t n_nodes, int na
 }
 
 // ---- level 0 on a lattice: per-node matrix-free operator -------------------
+// For congruent cells that are no axis-aligned boxes (lattice_box.hip has those).
 // Thread per lattice point n, vectors component-major in lattice order (x
 // fastest), so each neighbour gather of a wave is one contiguous 512-byte run;
 // work-groups in XCD-aware order; for each existing cell at n
@@ -787,48 +787,38 @@ __global__ __launch_bounds__(256) void k_lattice_apply(CGArgs C, const double* _
     block_sum_store(dsum, C.part0, blockIdx.x);
 }
 
-// Chebyshev epilogue of one DOF of the FP32 problem-level state (see mg_epilogue)
-__device__ __forceinline__ void mg_epilogue32(const MGLevelArgs& L, int mode, int64_t i, float y,
-                                              const float* __restrict__ din, float* __restrict__ dout, float c1,
-                                              float c2, float ith) {
-    if (mode == MG_RESID_INIT) {
-        const float rs = float(L.r[i]) - y;
-        L.res32[i] = rs;
-        dout[i] = L.dinv32[i] * rs * ith;
-    } else {
-        const float dv = din[i];
-        L.x32[i] += dv;
-        const float rs = L.res32[i] - y;
-        L.res32[i] = rs;
-        if (mode == MG_STEP) dout[i] = c1 * dv + c2 * L.dinv32[i] * rs;
-    }
-}
-
-// Multigrid smoothing step on the hex8 problem level in FP32: the lattice
-// operator on the FP32 direction (MG_RESID_INIT: on the iterate) with the
-// row-local Chebyshev epilogue.  The smoother is part of the preconditioner;
-// the CG operator, its residuals and the convergence test stay FP64.
-__global__ __launch_bounds__(256) void k_lattice_smooth(LatticeOpArgs O, MGLevelArgs L, int mode, int step,
-                                                        const float* __restrict__ din, float* __restrict__ dout,
-                                                        const int* __restrict__ done) {
+// One pass of the hex8 problem level's FP32 smoothing (LatSmooth).  The
+// smoother is part of the preconditioner; the CG operator, its residuals and
+// the convergence test stay FP64.  The last work-group, if S.check, only decides
+// on convergence.
+__global__ __launch_bounds__(256) void k_lattice_smooth(LatticeOpArgs O, LatSmooth S, const int* __restrict__ done) {
     if (done && *done) return;
+    unsigned nb = gridDim.x;
+    if (S.check.S) {
+        nb--;
+        if (blockIdx.x == nb) {
+            pcg_check_block(S.check);
+            return;
+        }
+    }
     const int64_t n_lat = int64_t(O.nx + 1) * (O.ny + 1) * (O.nz + 1);
-    const int64_t p = xcd_block(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
-    if (p >= n_lat) return;   // no block-level synchronisation below
-    const float* __restrict__ in = mode == MG_RESID_INIT ? L.x32 : din;
+    const int64_t t = xcd_block(blockIdx.x, nb) * 256 + threadIdx.x, p = t < n_lat ? t : 0;
     int i, j, k, cnt;
     lattice_point(O, p, i, j, k);
-    float y0, y1, y2;
-    lattice_row<float>(O, in, O.Khat32, n_lat, i, j, k, true, y0, y1, y2, cnt);
+    float y[3];
+    lattice_row<float>(O, S.x, O.Khat32, n_lat, i, j, k, true, y[0], y[1], y[2], cnt);
     const int m = O.nodecon[p];
-    if (m & 1) y0 = float(cnt) * in[p];
-    if (m & 2) y1 = float(cnt) * in[p + n_lat];
-    if (m & 4) y2 = float(cnt) * in[p + 2 * n_lat];
-    const float ith = float(L.cheb[0]);
-    const float c1 = step > 0 ? float(L.cheb[2 * step]) : 0.f, c2 = step > 0 ? float(L.cheb[2 * step + 1]) : 0.f;
-    mg_epilogue32(L, mode, p, y0, din, dout, c1, c2, ith);
-    mg_epilogue32(L, mode, p + n_lat, y1, din, dout, c1, c2, ith);
-    mg_epilogue32(L, mode, p + 2 * n_lat, y2, din, dout, c1, c2, ith);
+    const LatCoef cf = lat_coef(S);
+    double rz = 0.0;
+    if (t < n_lat)
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            const int64_t q = c * n_lat + p;
+            const float x = S.x[q];
+            rz += lat_point(S, cf, q, (m >> c) & 1 ? float(cnt) * x : y[c], x, S.b[q], S.res ? 0.f : S.dinv[q],
+                            S.xp ? S.xp[q] : 0.f);
+        }
+    if (S.part) block_sum_store(rz, S.part, blockIdx.x);
 }
 
 // Row information of the lattice operator without an assembled matrix: for
@@ -1320,12 +1310,18 @@ __global__ __launch_bounds__(256) void k_pcg_update(CGArgs C) {
     block_sum_store(rr, C.part1, blockIdx.x);
 }
 
-// the same update, with the start of the hex8 problem level's FP32
-// pre-smoothing (x = 0, res = r, first direction D^-1 r / theta) written from
-// the updated residual (the V-cycle's own start kernel is then skipped)
-__global__ __launch_bounds__(256) void k_pcg_update_mg(CGArgs C, MGLevelArgs L) {
-    if (C.S->done) return;
-    const double a = C.S->alpha;
+// the lattice solver's update: every work-group sums the operator's partials
+// of p.q itself (a launch less than a kernel for alpha); x, r, the partials of
+// r.r, and the start of the FP32 pre-smoothing (b = r, x = D^-1 b / theta)
+__global__ __launch_bounds__(256) void k_pcg_update_lat(CGArgs C, MGLevelArgs L) {
+    CGScalars* S = C.S;
+    if (S->done) return;
+    const double pq = reduce_partials(C.part0, C.nparts_op);
+    if (!(pq > 0.0) || !isfinite(pq)) {   // breakdown / NaN, the same in every work-group
+        if (blockIdx.x == 0 && threadIdx.x == 0) S->done = 3;
+        return;
+    }
+    const double a = S->rz2[S->iter & 1] / pq;
     const float ith = float(L.cheb[0]);
     double rr = 0.0;
     for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < C.n; i += int64_t(gridDim.x) * 256) {
@@ -1334,25 +1330,33 @@ __global__ __launch_bounds__(256) void k_pcg_update_mg(CGArgs C, MGLevelArgs L) 
         C.r[i] = r;
         rr += r * r;
         const float rf = float(r);
-        L.x32[i] = 0.f;
-        L.res32[i] = rf;
-        L.da32[i] = L.dinv32[i] * rf * ith;
+        L.b32[i] = rf;
+        L.x32[i] = L.dinv32[i] * rf * ith;
     }
     block_sum_store(rr, C.part1, blockIdx.x);
+}
+
+// r.z summed by every work-group, beta = r.z / the last r.z, p = z + beta p
+// (first: p = z); a non-positive r.z means the preconditioner is not SPD
+__global__ __launch_bounds__(256) void k_pcg_p_lat(CGArgs C, const float* __restrict__ z, int n, int first) {
+    CGScalars* S = C.S;
+    if (S->done) return;
+    const double rz = reduce_partials(C.part0, n);
+    const int it = S->iter;
+    if (!(rz > 0.0) || !isfinite(rz)) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) S->done = 3;
+        return;
+    }
+    const double beta = first ? 0.0 : rz / S->rz2[(it + 1) & 1];
+    if (blockIdx.x == 0 && threadIdx.x == 0) S->rz2[it & 1] = rz;
+    for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < C.n; i += int64_t(gridDim.x) * 256)
+        C.p[i] = first ? double(z[i]) : double(z[i]) + beta * C.p[i];
 }
 
 // convergence on the updated residual, before the V-cycle runs
 __global__ __launch_bounds__(256) void k_pcg_check(CGArgs C) {
     if (C.S->done) return;
-    const double rr = reduce_partials(C.part1, C.nvec);
-    if (threadIdx.x == 0) {
-        CGScalars* S = C.S;
-        S->rr = rr;
-        S->iter += 1;
-        if (!isfinite(rr)) S->done = 4;
-        else if (rr <= S->tol2 * S->bb) S->done = 1;
-        else if (S->iter >= S->max_it) S->done = 2;
-    }
+    pcg_check_block(CGCheck{C.S, C.part1, C.nvec});
 }
 
 // z = x0 + dlast (the level-0 V-cycle output) ; partials r.z
@@ -1362,18 +1366,6 @@ __global__ __launch_bounds__(256) void k_pcg_rz(CGArgs C, const double* __restri
     double rz = 0.0;
     for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < C.n; i += int64_t(gridDim.x) * 256) {
         const double z = dlast ? x0[i] + dlast[i] : x0[i];
-        C.z[i] = z;
-        rz += C.r[i] * z;
-    }
-    block_sum_store(rz, C.part0, blockIdx.x);
-}
-
-__global__ __launch_bounds__(256) void k_pcg_rz32(CGArgs C, const float* __restrict__ x0,
-                                                  const float* __restrict__ dlast) {
-    if (C.S->done) return;
-    double rz = 0.0;
-    for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < C.n; i += int64_t(gridDim.x) * 256) {
-        const double z = dlast ? double(x0[i] + dlast[i]) : double(x0[i]);
         C.z[i] = z;
         rz += C.r[i] * z;
     }
@@ -1524,16 +1516,24 @@ void launch_mg_power(const MGLevelArgs& L, const double* val, int n_it, double s
         out = out == w0 ? w1 : w0;
     }
 }
-int64_t lattice_partials(const LatticeOpArgs& l) {
+static int64_t lattice_blocks(const LatticeOpArgs& l) {
     return (int64_t(l.nx + 1) * (l.ny + 1) * (l.nz + 1) + 255) / 256;
 }
+int64_t lattice_partials(const LatticeOpArgs& l) { return l.is_box ? box_partials(l) : lattice_blocks(l); }
+int64_t lattice_partials_most(const LatticeOpArgs& l) { return std::max(lattice_blocks(l), box_partials_most(l)); }
 void launch_lattice_apply(const CGArgs& c, const double* x, double* y, hipStream_t s) {
     const int* done = c.S ? &c.S->done : nullptr;
-    hipLaunchKernelGGL(k_lattice_apply, dim3(unsigned(lattice_partials(c.lat))), dim3(256), 0, s, c, x, y, done);
+    if (c.lat.is_box) return launch_box_apply(c.lat, x, y, c.part0, done, s);
+    hipLaunchKernelGGL(k_lattice_apply, dim3(unsigned(lattice_blocks(c.lat))), dim3(256), 0, s, c, x, y, done);
+}
+void launch_lattice_smooth(const LatticeOpArgs& l, const LatSmooth& S, const int* done, hipStream_t s) {
+    if (l.is_box) return launch_box_smooth(l, S, done, s);
+    hipLaunchKernelGGL(k_lattice_smooth, dim3(unsigned(lattice_blocks(l)) + (S.check.S ? 1 : 0)), dim3(256), 0, s, l, S,
+                       done);
 }
 void launch_lattice_rowinfo(const LatticeOpArgs& l, double* dinv, float* dinv32, double* part, double* lam,
                             hipStream_t s) {
-    const int nb = int(lattice_partials(l));
+    const int nb = int(lattice_blocks(l));
     hipLaunchKernelGGL(k_lattice_rowinfo, dim3(nb), dim3(256), 0, s, l, dinv, dinv32, part);
     hipLaunchKernelGGL(k_mg_max, dim3(1), dim3(256), 0, s, part, nb, lam);
 }
@@ -1637,11 +1637,6 @@ void launch_mg_bsr(const MGLevelArgs& L, int mode, int step, const double* din, 
             hipLaunchKernelGGL((k_mg_bsr<double, 3>), dim3(g), dim3(256), 0, s, L, L.val, mode, step, din, dout, done);
     }
 }
-void launch_mg_fine(const CGArgs& c, const MGLevelArgs& L, int mode, int step, const float* din, float* dout,
-                    const int* done, hipStream_t s) {
-    hipLaunchKernelGGL(k_lattice_smooth, dim3(unsigned(lattice_partials(c.lat))), dim3(256), 0, s, c.lat, L, mode,
-                       step, din, dout, done);
-}
 void launch_mg_restrict(const MGLevelArgs& F, const MGLevelArgs& C, const int* done, hipStream_t s) {
     const dim3 g(mg_blocks(C.n_nodes, 256));
     const int fl = F.planar ? FL_PLANAR : F.rank_of_lat ? FL_RANK : FL_LAT;
@@ -1683,15 +1678,14 @@ void launch_pcg_update(const CGArgs& c, hipStream_t s) {
     hipLaunchKernelGGL(k_pcg_update, dim3(c.nvec), dim3(256), 0, s, c);
     hipLaunchKernelGGL(k_pcg_check, dim3(1), dim3(256), 0, s, c);
 }
-void launch_pcg_update_mg(const CGArgs& c, const MGLevelArgs& L, hipStream_t s) {
-    hipLaunchKernelGGL(k_pcg_update_mg, dim3(c.nvec), dim3(256), 0, s, c, L);
-    hipLaunchKernelGGL(k_pcg_check, dim3(1), dim3(256), 0, s, c);
+void launch_pcg_update_lat(const CGArgs& c, const MGLevelArgs& L, hipStream_t s) {
+    hipLaunchKernelGGL(k_pcg_update_lat, dim3(c.nvec), dim3(256), 0, s, c, L);
+}
+void launch_pcg_p_lat(const CGArgs& c, const float* z, int n, int first, hipStream_t s) {
+    hipLaunchKernelGGL(k_pcg_p_lat, dim3(c.nvec), dim3(256), 0, s, c, z, n, first);
 }
 void launch_pcg_rz(const CGArgs& c, const double* x0, const double* dlast, hipStream_t s) {
     hipLaunchKernelGGL(k_pcg_rz, dim3(c.nvec), dim3(256), 0, s, c, x0, dlast);
-}
-void launch_pcg_rz32(const CGArgs& c, const float* x0, const float* dlast, hipStream_t s) {
-    hipLaunchKernelGGL(k_pcg_rz32, dim3(c.nvec), dim3(256), 0, s, c, x0, dlast);
 }
 void launch_mg_combine(int64_t n, const double* x0, const double* dlast, double* out, const int* done,
                        hipStream_t s) {
