@@ -943,11 +943,11 @@ int mg_build(mastg_ctx* c) {
     }
     TRY(dalloc(c, c->mg_cheb, size_t(nl) * kMGChebStride * sizeof(double)));
     TRY(dalloc(c, c->mg_lam, size_t(nl) * sizeof(double)));
-    TRY(dalloc(c, c->mg_part, size_t(std::max<int64_t>(8192, (c->S.n_active + 255) / 256 + 1)) * sizeof(double)));
+    TRY(dalloc(c, c->mg_part, size_t(std::max<int64_t>({8192, (c->S.n_active + 255) / 256 + 1, mg_power_partials(nl)})) *
+                                  sizeof(double)));
     c->mg_n_coarse = H.coarsest_dofs;
     TRY(dalloc(c, c->mg_dense, size_t(H.coarsest_dofs * H.coarsest_dofs) * sizeof(double)));
     TRY(dalloc(c, c->mg_dense_w, size_t(mg_invert_work(int(H.coarsest_dofs))) * sizeof(double)));
-    TRY(dalloc(c, c->mg_scal, 2 * sizeof(double)));
     // plates: the Gershgorin bound of D^-1 A is loose by ~50x (thin-plate
     // bending against membrane rows); their Chebyshev intervals come from
     // power iteration instead (heat too: its Jacobian is not symmetric)
@@ -970,6 +970,14 @@ int mg_setup(mastg_ctx* c) {
     const int nav = c->S.nav;
     hipStream_t s = c->stream;
     MGLevelDev& L0 = *c->mg[0];
+    // levels whose Chebyshev bound comes from power iteration, run together
+    // once all of them are formed
+    MGPowerArgs P{};
+    P.nav = nav;
+    P.part = c->mg_part.as<double>();
+    auto power_level = [&](const MGLevelArgs& a, int l) {
+        P.level[P.n++] = {a.n_nodes, a.blk_ptr, a.blk_col, a.val, a.dinv, a.dinvb, a.da, a.db, c->mg_lam.as<double>() + l};
+    };
     if (lat) {
         ensure_scales(c);
         CGArgs la = cg_args(c);
@@ -1019,8 +1027,7 @@ int mg_setup(mastg_ctx* c) {
             L0.a.rs16 = L0.srow16.as<float>();
         } else {
             if (L0.a.dinvb) launch_mg_block_dinv5(L0.a, L0.dinvb.as<float>(), s);
-            launch_mg_power(L0.a, c->val.as<double>(), kMGPowerIters, kMGPowerSafety, L0.a.da, L0.a.db,
-                            c->mg_part.as<double>(), c->mg_scal.as<double>(), c->mg_lam.as<double>(), s);
+            power_level(L0.a, 0);
         }
     }
     for (int l = 0; l + 1 < nl; l++) {
@@ -1061,10 +1068,12 @@ int mg_setup(mastg_ctx* c) {
         // 104 with 20-step power iterations on every level of every Newton
         // step's hierarchy); plates (a loose Gershgorin bound) and hex8 on
         // cells of several shapes (2 PCG iterations fewer than with the
-        // Gershgorin bound at 128 x 64 x 64): power iteration
-        if (c->d.physics != MASTG_HEX8_HEAT)
-            launch_mg_power(C.a, C.a.val, kMGPowerIters, kMGPowerSafety, C.a.da, C.a.db, c->mg_part.as<double>(),
-                            c->mg_scal.as<double>(), c->mg_lam.as<double>() + l + 1, s);
+        // Gershgorin bound at 128 x 64 x 64): power iteration; hex8 on one
+        // cell shape: power iteration too, except on the first coarse level,
+        // where the 20 products cost more than the iteration they save
+        // (128x64x64: 0.8 ms; 19-20 iterations either way, 20 with Gershgorin
+        // bounds on every level, and 1-2 more on smaller meshes)
+        if (nav != 1 && (!lat || l > 0)) power_level(C.a, l + 1);
         launch_to_f32(int64_t(C.val32.bytes / sizeof(float)), C.a.val, C.val32.as<float>(), s);
         if (nav == 5 && l == 0) {
             // the plate's first coarse level smooths in FP16 too (row scales)
@@ -1079,6 +1088,7 @@ int mg_setup(mastg_ctx* c) {
             else launch_mg_to_stencil(C.a, C.sten.as<float>(), s);
         }
     }
+    launch_mg_power(P, kMGPowerIters, kMGPowerSafety, s);
     // hex8 cells of several shapes (assembled problem level): [lam/30, lam]
     // (33 iterations at 3 steps on the distorted 128x64x64 against 35 at the
     // lattice's 80; 20 and 45 the same as 30)

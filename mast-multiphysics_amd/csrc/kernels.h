@@ -418,11 +418,6 @@ void launch_mg_stencil_rank(const MGLevelArgs& L, const float* sten, int mode, i
                             double* dout, const int* done, hipStream_t s);
 void launch_perm_rank_lat(int64_t n_nodes, int nav, const int32_t* rank_of_lat, const double* src, double* dst,
                           int to_lat, const int* done, hipStream_t s);
-// lambda_max(D^-1 A) of the heat problem level by power iteration on its
-// lattice-ordered stencil (L: the level in lattice order, its inverse diagonal)
-void launch_mg_power_heat(const MGLevelArgs& L, const float* sten, const int32_t* rank_of_lat, int n_it,
-                          double safety, double* w0, double* w1, double* part, double* scal, double* lam,
-                          hipStream_t s);
 void launch_mg_combine_rank(int64_t n_nodes, int nav, const int32_t* rank_of_lat, const double* x0,
                             const double* dlast, double* out, const int* done, hipStream_t s);
 void launch_mg_to_stencil(const MGLevelArgs& L, float* sten, hipStream_t s);
@@ -453,11 +448,27 @@ void launch_perm_nodes(int64_t n_nodes, const int32_t* map, const double* src, d
                        hipStream_t s);
 void launch_mg_rowinfo_nb(int nav, int64_t n_nodes, const int64_t* blk_ptr, const int32_t* blk_col,
                           const double* val, double* dinv, double* part, double* lam, hipStream_t s);
-// estimate of lambda_max(D^-1 A) by power iteration on the FP64 node blocks of
-// L (n_it steps from a fixed positive start vector), times `safety`, into
-// *lam; w0, w1: work vectors of nav n_nodes; scal: 2 device doubles
-void launch_mg_power(const MGLevelArgs& L, const double* val, int n_it, double safety, double* w0, double* w1,
-                     double* part, double* scal, double* lam, hipStream_t s);
+// estimates of lambda_max(D^-1 A) by power iteration on the FP64 node blocks of
+// the n levels of P (n_it steps from a fixed positive start vector), times
+// `safety`, into their *lam; w0, w1: work vectors of nav n_nodes; part:
+// mg_power_partials(n) doubles; nav 3 or 5
+constexpr int kMGMaxLevels = 16;
+struct MGPowerLevel {
+    int64_t n_nodes;
+    const int64_t* blk_ptr;
+    const int32_t* blk_col;
+    const double *val, *dinv;
+    const float* dinvb;                // (plate problem level) block Jacobi, or null
+    double *w0, *w1, *lam;
+};
+struct MGPowerArgs {
+    int n, nav;
+    double* part;
+    MGPowerLevel level[kMGMaxLevels];
+    int first[kMGMaxLevels + 1];       // set by the launcher
+};
+int64_t mg_power_partials(int n_levels);
+void launch_mg_power(MGPowerArgs P, int n_it, double safety, hipStream_t s);
 void launch_mg_restrict(const MGLevelArgs& F, const MGLevelArgs& C, const int* done, hipStream_t s);
 // (F planar: the fine vectors are F's FP32 state)
 void launch_mg_prolong(const MGLevelArgs& F, const MGLevelArgs& C, const double* dlast, const int* done,

@@ -586,38 +586,6 @@ __global__ __launch_bounds__(256) void k_mg_stencil_heat(MGLevelArgs L, const T*
     mg_epilogue(L, mode, p, y, din, dout, c1, c2, ith);
 }
 
-// power iteration for lambda_max(D^-1 A) on the heat problem level in lattice
-// order with its stencil: out = D^-1 A (s in), s = *scale; the start vector
-// (in == null) is the rank-ordered one, 1 + ((rank 7919) mod 1000) / 1000, read
-// through rank_of_lat, so the iterates are those of the node-block form
-// permuted; partial sums of out.out per work-group
-__global__ __launch_bounds__(256) void k_mg_power_heat(MGLevelArgs L, const float* __restrict__ sten,
-                                                       const int32_t* __restrict__ rank_of_lat,
-                                                       const double* __restrict__ in, const double* __restrict__ scale,
-                                                       double* __restrict__ out, double* __restrict__ part) {
-    const int64_t p = int64_t(blockIdx.x) * 256 + threadIdx.x;
-    double acc = 0.0;
-    if (p < L.n_nodes) {
-        const int64_t N = L.n_nodes;
-        const double sc = in ? *scale : 1.0;
-        const uint32_t nxp = uint32_t(L.nx + 1), nyp = uint32_t(L.ny + 1), pu = uint32_t(p), pq = pu / nxp;
-        const int i = int(pu - pq * nxp), j = int(pq % nyp), k = int(pq / nyp);
-        double y = 0.0;
-#pragma unroll 9
-        for (int o = 0; o < 27; o++) {
-            const int ni = min(max(i + o % 3 - 1, 0), L.nx), nj = min(max(j + (o / 3) % 3 - 1, 0), L.ny),
-                      nk = min(max(k + o / 9 - 1, 0), L.nz);
-            const int64_t m = int64_t(uint32_t(ni) + nxp * (uint32_t(nj) + nyp * uint32_t(nk)));
-            const double x = in ? sc * in[m] : 1.0 + double((int64_t(rank_of_lat[m]) * 7919) % 1000) / 1000.0;
-            y = fma(double(sten[o * N + p]), x, y);
-        }
-        const double o = L.dinv[p] * y;
-        out[p] = o;
-        acc = o * o;
-    }
-    block_sum_store(acc, part, blockIdx.x);
-}
-
 // node-major vectors between rank order and lattice order: to_lat = 1:
 // dst[p nav + v] = src[rank_of_lat[p] nav + v], else the inverse scatter
 __global__ __launch_bounds__(256) void k_perm_rank_lat(int64_t n_nodes, int nav, const int32_t* __restrict__ rank_of_lat,
@@ -951,21 +919,16 @@ __global__ __launch_bounds__(256) void k_mg_rowinfo_nb(int64_t n_nodes, const in
     block_max_store(g, part, blockIdx.x);
 }
 
-// power iteration for lambda_max(D^-1 A): out = D^-1 A (s in), s = *scale
-// (1 / ||in||; the start vector is built in place when in == null), with
-// partial sums of out.out
+// the rows of one level in a power step, 8 lanes per node
 template <int NAV>
-__global__ __launch_bounds__(256) void k_mg_power(MGLevelArgs L, const double* __restrict__ val,
-                                                  const double* __restrict__ in, const double* __restrict__ scale,
-                                                  double* __restrict__ out, double* __restrict__ part) {
+__device__ __forceinline__ void mg_power_rows(const MGPowerLevel& L, const double* __restrict__ in, double sc,
+                                              bool start, double* __restrict__ out, double* part, int blk, int nblk) {
     const int sub = threadIdx.x & 7;
-    const double sc = in ? *scale : 1.0;
     double acc = 0.0;
-    const int64_t nodes_per_grid = (int64_t(gridDim.x) * 256) / 8;
-    for (int64_t r = (int64_t(blockIdx.x) * 256 + threadIdx.x) / 8; r < L.n_nodes; r += nodes_per_grid) {
+    for (int64_t r = (int64_t(blk) * 256 + threadIdx.x) / 8; r < L.n_nodes; r += int64_t(nblk) * 32) {
         const int64_t k0 = L.blk_ptr[r];
         const int deg = int(L.blk_ptr[r + 1] - k0);
-        const double* __restrict__ V = val + k0 * (NAV * NAV);
+        const double* __restrict__ V = L.val + k0 * (NAV * NAV);
         double sv[NAV];
 #pragma unroll
         for (int v = 0; v < NAV; v++) sv[v] = 0.0;
@@ -973,8 +936,8 @@ __global__ __launch_bounds__(256) void k_mg_power(MGLevelArgs L, const double* _
             const int64_t cb = int64_t(L.blk_col[k0 + k]) * NAV;
             double xw[NAV];
 #pragma unroll
-            for (int w = 0; w < NAV; w++)   // start vector 1 + ((i * 7919) mod 1000) / 1000
-                xw[w] = in ? sc * in[cb + w] : 1.0 + double(((cb + w) * 7919) % 1000) / 1000.0;
+            for (int w = 0; w < NAV; w++)
+                xw[w] = start ? 1.0 + double(((cb + w) * 7919) % 1000) / 1000.0 : sc * in[cb + w];
 #pragma unroll
             for (int v = 0; v < NAV; v++) {
                 const double* vr = V + (int64_t(v) * deg + k) * NAV;
@@ -999,37 +962,38 @@ __global__ __launch_bounds__(256) void k_mg_power(MGLevelArgs L, const double* _
                 acc += o * o;
             }
     }
-    block_sum_store(acc, part, blockIdx.x);
+    block_sum_store(acc, part, blk);
 }
 
-// norm of the power iterate: scal[0] = 1 / ||out||, *lam = safety * ||out|| / ||start||
-__global__ __launch_bounds__(256) void k_mg_power_norm(const double* __restrict__ part, int n, int first,
-                                                       double safety, double* __restrict__ scal,
-                                                       double* __restrict__ lam) {
-    const double s = reduce_partials(part, n);
-    if (threadIdx.x == 0) {
-        const double nrm = sqrt(s);
-        // the first step multiplies the unnormalised start vector: its norm is scal[1]
-        const double rel = first ? nrm / scal[1] : nrm;
-        scal[0] = nrm > 0.0 ? 1.0 / nrm : 0.0;
-        *lam = safety * rel;
+// Power iteration for lambda_max(D^-1 A) of several levels at once: one step of
+// every level per launch (work-groups [first[l], first[l + 1]) take level l),
+// out = D^-1 A (in / ||in||), ||in||^2 summed by every work-group from the
+// partials the step before left, partial sums of out.out.  The start vector
+// (step 0) is 1 + ((i 7919) mod 1000) / 1000.  Level by level, with a kernel for
+// each norm, the 20 steps were 42 launches per level of 5-7 us each (64x64
+// plate: 0.9 ms for 5 levels, now 0.15 ms).
+__global__ __launch_bounds__(256) void k_mg_power(MGPowerArgs P, int step) {
+    int l = 0;
+    while (int(blockIdx.x) >= P.first[l + 1]) l++;
+    const MGPowerLevel& L = P.level[l];
+    const int blk = blockIdx.x - P.first[l], nblk = P.first[l + 1] - P.first[l];
+    const double* __restrict__ in = step & 1 ? L.w0 : L.w1;
+    double* __restrict__ out = step & 1 ? L.w1 : L.w0;
+    double* part = P.part + P.first[l] + (step & 1 ? P.first[P.n] : 0);
+    double sc = 1.0;
+    if (step > 0) {
+        const double s = reduce_partials(P.part + P.first[l] + (step & 1 ? 0 : P.first[P.n]), nblk);
+        sc = s > 0.0 ? 1.0 / sqrt(s) : 0.0;
     }
+    if (P.nav == 5) mg_power_rows<5>(L, in, sc, step == 0, out, part, blk, nblk);
+    else mg_power_rows<3>(L, in, sc, step == 0, out, part, blk, nblk);
 }
 
-// squared norm of the start vector (for the first Rayleigh-free estimate)
-__global__ __launch_bounds__(256) void k_mg_power_start(int64_t n, double* __restrict__ part) {
-    double acc = 0.0;
-    for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < n; i += int64_t(gridDim.x) * 256) {
-        const double x = 1.0 + double((i * 7919) % 1000) / 1000.0;
-        acc += x * x;
-    }
-    block_sum_store(acc, part, blockIdx.x);
-}
-
-__global__ __launch_bounds__(256) void k_mg_power_start_norm(const double* __restrict__ part, int n,
-                                                             double* __restrict__ scal) {
-    const double s = reduce_partials(part, n);
-    if (threadIdx.x == 0) scal[1] = sqrt(s);
+// lam[l] = safety ||out|| of the last step (its input had norm 1)
+__global__ __launch_bounds__(256) void k_mg_power_lam(MGPowerArgs P, int last, double safety) {
+    const int l = blockIdx.x;
+    const double s = reduce_partials(P.part + P.first[l] + (last & 1 ? P.first[P.n] : 0), P.first[l + 1] - P.first[l]);
+    if (threadIdx.x == 0) *P.level[l].lam = safety * sqrt(s);
 }
 
 // ---- transfers ---------------------------------------------------------------
@@ -1496,25 +1460,16 @@ void launch_mg_rowinfo_nb(int nav, int64_t n_nodes, const int64_t* blk_ptr, cons
         hipLaunchKernelGGL(k_mg_rowinfo_nb<3>, dim3(nb), dim3(256), 0, s, n_nodes, blk_ptr, blk_col, val, dinv, part);
     hipLaunchKernelGGL(k_mg_max, dim3(1), dim3(256), 0, s, part, nb, lam);
 }
-void launch_mg_power(const MGLevelArgs& L, const double* val, int n_it, double safety, double* w0, double* w1,
-                     double* part, double* scal, double* lam, hipStream_t s) {
-    const int nb = nb_grid(L.n_nodes);
-    const int nbs = int(std::min<int64_t>(mg_blocks(L.n_nodes * L.nav, 256), 8192));
-    hipLaunchKernelGGL(k_mg_power_start, dim3(nbs), dim3(256), 0, s, L.n_nodes * L.nav, part);
-    hipLaunchKernelGGL(k_mg_power_start_norm, dim3(1), dim3(256), 0, s, part, nbs, scal);
-    double* in = nullptr;
-    double* out = w0;
-    for (int it = 0; it < n_it; it++) {
-        if (L.nav == 5)
-            hipLaunchKernelGGL(k_mg_power<5>, dim3(nb), dim3(256), 0, s, L, val, in, scal, out, part);
-        else if (L.nav == 1)
-            hipLaunchKernelGGL(k_mg_power<1>, dim3(nb), dim3(256), 0, s, L, val, in, scal, out, part);
-        else
-            hipLaunchKernelGGL(k_mg_power<3>, dim3(nb), dim3(256), 0, s, L, val, in, scal, out, part);
-        hipLaunchKernelGGL(k_mg_power_norm, dim3(1), dim3(256), 0, s, part, nb, it == 0 ? 1 : 0, safety, scal, lam);
-        in = out;
-        out = out == w0 ? w1 : w0;
-    }
+// work-groups of a level: enough for its rows, at most kPowerBlocks (each sums
+// all the level's partials)
+constexpr int kPowerBlocks = 1024;
+int64_t mg_power_partials(int n_levels) { return 2 * int64_t(n_levels) * kPowerBlocks; }
+void launch_mg_power(MGPowerArgs P, int n_it, double safety, hipStream_t s) {
+    if (P.n <= 0) return;
+    P.first[0] = 0;
+    for (int l = 0; l < P.n; l++) P.first[l + 1] = P.first[l] + std::min(nb_grid(P.level[l].n_nodes), kPowerBlocks);
+    for (int it = 0; it < n_it; it++) hipLaunchKernelGGL(k_mg_power, dim3(P.first[P.n]), dim3(256), 0, s, P, it);
+    hipLaunchKernelGGL(k_mg_power_lam, dim3(P.n), dim3(256), 0, s, P, n_it - 1, safety);
 }
 static int64_t lattice_blocks(const LatticeOpArgs& l) {
     return (int64_t(l.nx + 1) * (l.ny + 1) * (l.nz + 1) + 255) / 256;
@@ -1581,22 +1536,6 @@ void launch_mg_stencil_rank(const MGLevelArgs& L, const float* sten, int mode, i
 }
 void launch_sten27_to_f16(int64_t n, const float* sten, uint16_t* sten16, float* srow, hipStream_t s) {
     hipLaunchKernelGGL(k_sten27_to_f16, dim3(unsigned((n + 255) / 256)), dim3(256), 0, s, n, sten, sten16, srow);
-}
-void launch_mg_power_heat(const MGLevelArgs& L, const float* sten, const int32_t* rank_of_lat, int n_it,
-                          double safety, double* w0, double* w1, double* part, double* scal, double* lam,
-                          hipStream_t s) {
-    const int nb = int(mg_blocks(L.n_nodes, 256));
-    const int nbs = int(std::min<int64_t>(mg_blocks(L.n_nodes, 256), 8192));
-    hipLaunchKernelGGL(k_mg_power_start, dim3(nbs), dim3(256), 0, s, L.n_nodes, part);
-    hipLaunchKernelGGL(k_mg_power_start_norm, dim3(1), dim3(256), 0, s, part, nbs, scal);
-    double* in = nullptr;
-    double* out = w0;
-    for (int it = 0; it < n_it; it++) {
-        hipLaunchKernelGGL(k_mg_power_heat, dim3(nb), dim3(256), 0, s, L, sten, rank_of_lat, in, scal, out, part);
-        hipLaunchKernelGGL(k_mg_power_norm, dim3(1), dim3(256), 0, s, part, nb, it == 0 ? 1 : 0, safety, scal, lam);
-        in = out;
-        out = out == w0 ? w1 : w0;
-    }
 }
 void launch_perm_rank_lat(int64_t n_nodes, int nav, const int32_t* rank_of_lat, const double* src, double* dst,
                           int to_lat, const int* done, hipStream_t s) {
