@@ -111,6 +111,7 @@ struct MGLevelDev {
     DevBuf sten16, srow16;        // heat level 0: the stencil in FP16 and its row scales; plate
                                   // level 1: its node blocks in FP16 and their row scales
     bool lat0 = false;            // heat / hex8 level 0 smooths in lattice order
+    DevBuf tail;                  // levels of the one-launch tail: their entries by offset
     DevBuf Kel, val, val32, dinv, r, x, res, da, db;
 };
 
@@ -180,7 +181,8 @@ struct mastg_ctx {
     bool mg_k0_set = false;    // problem-level steps chosen by the caller (MASTG_OPT_MG_STEPS_FINE)
     int mg_ratio = 0;          // Chebyshev interval [lam / ratio, lam] (0: the physics' default)
     int64_t mg_n_coarse = 0;   // DOFs of the dense coarsest level
-    DevBuf mg_cheb, mg_lam, mg_part, mg_dense, mg_dense_w, mg_scal;
+    int mg_tail = 0;           // first level of the V-cycle's one-launch tail (the level count: none)
+    DevBuf mg_cheb, mg_lam, mg_part, mg_dense, mg_dense_w;
     bool mg_power = false;     // Chebyshev bounds from power iteration (plates)
     hipGraphExec_t mg_exec = nullptr;
     int mg_exec_len = 0;
@@ -902,9 +904,21 @@ int mg_build(mastg_ctx* c) {
         }
         lv.push_back(std::move(L));
     }
-    if (c->d.physics == MASTG_HEX8_HEAT && nl > 2) {
+    // the levels one work-group holds
+    {
+        std::vector<MGTailLevel> tl(static_cast<size_t>(nl));
+        for (int l = 0; l < nl; l++) tl[l] = {H.levels[l].nx, H.levels[l].ny, H.levels[l].nz, int(H.levels[l].n_nodes)};
+        c->mg_tail = mg_tail_first(tl.data(), nl, c->S.nav);
+        if (c->mg_tail < nl) {
+            HipLock l(g_hip_mu);
+            HIPC(c, mg_tail_prepare());
+        }
+        for (int l = c->mg_tail; l + 1 < nl; l++)
+            TRY(dalloc(c, lv[l]->tail, size_t(mg_tail_entries(H.levels[l].dim, c->S.nav, H.levels[l].n_nodes)) * sizeof(float)));
+    }
+    if (c->d.physics == MASTG_HEX8_HEAT && std::min(nl - 1, c->mg_tail) > 1) {
         // heat: the first coarse level (lattice order) smooths with a 27-point
-        // stencil too when it is not the coarsest
+        // stencil too when it is above the tail and not the coarsest
         TRY(dalloc(c, lv[1]->sten, size_t(H.levels[1].n_nodes) * 27 * sizeof(float)));
     }
     if (!plate) {
@@ -938,8 +952,9 @@ int mg_build(mastg_ctx* c) {
         if (!list.empty()) TRY(upload(c, lv[1]->gal_list, list));
         lv[1]->n_dirty = int64_t(list.size());
         // the first coarse level smooths with its operator as a stencil
-        // (coalesced values, no column indices) when it is not the coarsest
-        if (nl > 2) TRY(dalloc(c, lv[1]->sten, size_t(H.levels[1].n_nodes) * 123 * sizeof(float)));
+        // (coalesced values, no column indices) when it is above the tail and
+        // not the coarsest
+        if (std::min(nl - 1, c->mg_tail) > 1) TRY(dalloc(c, lv[1]->sten, size_t(H.levels[1].n_nodes) * 123 * sizeof(float)));
     }
     TRY(dalloc(c, c->mg_cheb, size_t(nl) * kMGChebStride * sizeof(double)));
     TRY(dalloc(c, c->mg_lam, size_t(nl) * sizeof(double)));
@@ -1074,6 +1089,11 @@ int mg_setup(mastg_ctx* c) {
         // (128x64x64: 0.8 ms; 19-20 iterations either way, 20 with Gershgorin
         // bounds on every level, and 1-2 more on smaller meshes)
         if (nav != 1 && (!lat || l > 0)) power_level(C.a, l + 1);
+        if (C.tail.p) {   // smoothed by the tail alone, from its entries
+            launch_mg_tail_entries(C.a, C.tail.as<float>(), s);
+            continue;
+        }
+        if (l + 2 == nl) continue;   // the coarsest: its inverse reads the FP64 values
         launch_to_f32(int64_t(C.val32.bytes / sizeof(float)), C.a.val, C.val32.as<float>(), s);
         if (nav == 5 && l == 0) {
             // the plate's first coarse level smooths in FP16 too (row scales)
@@ -1188,7 +1208,8 @@ const void* mg_vcycle(mastg_ctx* c, const CGArgs& a, const int* done, hipStream_
                           done, s);
     };
     auto steps = [&](int l) { return l == 0 ? c->mg_k0 : c->mg_kc; };
-    for (int l = 0; l + 1 < nl; l++) {
+    const int lt = c->mg_tail;
+    for (int l = 0; l + 1 < nl && l < lt; l++) {
         const int k = steps(l);
         // coarse levels start their pre-smoothing inside the restriction
         if (l == 0 && !started) launch_mg_pre_init(lv(l), done, s);
@@ -1202,10 +1223,24 @@ const void* mg_vcycle(mastg_ctx* c, const CGArgs& a, const int* done, hipStream_
         }
         launch_mg_restrict(lv(l), lv(l + 1), done, s);
     }
-    const MGLevelArgs& Lc = lv(nl - 1);
-    launch_mg_coarse_solve(int(c->mg_n_coarse), c->mg_dense.as<double>(), Lc.r, Lc.x, done, s);
+    if (lt < nl) {
+        MGTailArgs T{};
+        T.n = nl - lt;
+        T.steps = c->mg_kc;
+        for (int l = lt; l < nl; l++) {
+            const MGLevelArgs& a = lv(l);
+            T.lv[l - lt] = {a.nx, a.ny, a.nz, int(a.n_nodes), c->mg[l]->tail.as<float>(), a.dinv, a.cheb, a.con};
+        }
+        T.Ainv = c->mg_dense.as<double>();
+        T.r = lv(lt).r;
+        T.x = lv(lt).x;
+        launch_mg_tail(T, L0.nav, done, s);
+    } else {
+        const MGLevelArgs& Lc = lv(nl - 1);
+        launch_mg_coarse_solve(int(c->mg_n_coarse), c->mg_dense.as<double>(), Lc.r, Lc.x, done, s);
+    }
     const double* dlast = nullptr;   // last direction of level l + 1 (coarse levels are FP64)
-    for (int l = nl - 2; l >= 0; l--) {
+    for (int l = std::min(lt, nl - 1) - 1; l >= 0; l--) {
         const int k = steps(l);
         launch_mg_prolong(lv(l), lv(l + 1), dlast, done, s);
         if (l == 0 && f32) {

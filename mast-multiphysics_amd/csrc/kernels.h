@@ -475,6 +475,27 @@ void launch_mg_prolong(const MGLevelArgs& F, const MGLevelArgs& C, const double*
                        hipStream_t s);
 void launch_mg_coarse_solve(int n, const double* Ainv, const double* r, double* x, const int* done,
                             hipStream_t s);
+// the coarse end of the V-cycle in one launch (mg_tail.hip): levels first ..
+// nl - 1 of a hierarchy (first = nl: none), every vector in one work-group's LDS
+constexpr int kMGTailLevels = 6;
+struct MGTailLevel {
+    int nx, ny, nz, n_nodes;
+    const float* ent;                  // entries by offset (null: the coarsest level)
+    const double *dinv, *cheb;
+    const uint8_t* con;
+};
+struct MGTailArgs {
+    int n, steps;                      // levels, Chebyshev steps per smoothing
+    MGTailLevel lv[kMGTailLevels];
+    const double *Ainv, *r;            // coarsest inverse; right side of the first level
+    double* x;                         // its result
+    int lds_doubles;                   // set by the launcher
+};
+int mg_tail_first(const MGTailLevel* lv, int nl, int nav);   // from the levels' sizes
+int64_t mg_tail_entries(int dim, int nav, int64_t n_nodes);
+hipError_t mg_tail_prepare();
+void launch_mg_tail_entries(const MGLevelArgs& L, float* ent, hipStream_t s);
+void launch_mg_tail(MGTailArgs A, int nav, const int* done, hipStream_t s);
 // preconditioned CG around the V-cycle
 void launch_pcg_update(const CGArgs& c, hipStream_t s);
 // the lattice solver's: alpha = r.z / p.q from the operator's partial sums, the

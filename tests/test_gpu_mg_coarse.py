@@ -1,6 +1,7 @@
 """The multigrid hierarchy's coarsest level: its blocked dense inverse at the
 edges of its 32 x 32 blocks (whole and partial last blocks, the smallest and
-the largest coarsest systems), through design evaluations at the bars every
+the largest coarsest systems), and the levels above it that one work-group
+runs, through design evaluations at the bars every
 solver meets (compliance 1e-9, gradient 1e-7 of the oracle's).  An inexact
 coarse solve would show as iterations: the bound is twice the V-cycle's usual
 count on these meshes."""
@@ -53,4 +54,58 @@ def test_coarsest_inverse_plate(oracle, mastg):
     assert r["rel_res"] <= 1.5e-10 and r["iters"] * 4 < ref["iters"], (r["iters"], ref["iters"])
     assert abs(r["objective"] - ref["compliance"]) <= 1e-9 * abs(ref["compliance"])
     assert rel_err_floor(r["grad"], ref["dc"], floor=1e-6) <= 1e-7
+    ctx.close()
+
+
+# The levels that one work-group runs: none above the dense one, one, several,
+# with a first level that nearly fills it or is just too large for it, and step
+# counts down to one (the first and last direction the same) and up to the most.
+@pytest.mark.parametrize("steps", [1, 2, 3, 8])
+@pytest.mark.parametrize("mesh", [
+    (16, 8, 8),      # 675 DOFs over 135
+    (24, 8, 8),      # 975 (of 1024 threads) over 189
+    (28, 8, 8),      # 1125 DOFs: too many, the separate kernels
+])
+def test_coarse_levels_hex8(oracle, mastg, mesh, steps):
+    print(f"[coarse levels] hex8 {mesh} steps {steps}", flush=True)
+    P = oracle.Problem(oracle.CANTILEVER, *mesh, seed=3, lo=0.1, hi=1.0)
+    ref = P.solve_elastic(1e-10)
+    ctx = ctx_from_oracle(mastg, P)
+    ctx.set_option(mastg.OPT_MG_STEPS_COARSE, steps)
+    r = ctx.design_eval(P.params(), solver=mastg.SOLVER_MG)
+    assert r["rel_res"] <= 1.5e-10 and r["iters"] * 2 < ref["iters"], (r["iters"], ref["iters"])
+    assert abs(r["objective"] - ref["compliance"]) <= 1e-9 * abs(ref["compliance"])
+    assert rel_err_floor(r["grad"], ref["dc"], floor=1e-6) <= 1e-7
+    ctx.close()
+
+
+@pytest.mark.parametrize("steps", [1, 2])
+@pytest.mark.parametrize("n", [16, 24])   # 729 over 125 DOFs; 2197 (three per thread) and 343 over 64
+def test_coarse_levels_heat(oracle, mastg, n, steps):
+    print(f"[coarse levels] heat {n}^3 steps {steps}", flush=True)
+    P = oracle.Problem(oracle.HEAT, n, seed=6)
+    ref = P.solve_heat(1e-12, 1e-14)
+    ctx = ctx_from_oracle(mastg, P)
+    ctx.set_option(mastg.OPT_MG_STEPS_COARSE, steps)
+    r = ctx.design_eval(P.params(), rtol=1e-12, solver=mastg.SOLVER_MG)
+    assert r["iters"] <= 30 * (r["newton_iters"] + 1), (r["iters"], r["newton_iters"])
+    assert abs(r["objective"] - ref["mean_T"]) <= 1e-9 * abs(ref["mean_T"])
+    assert rel_err_floor(r["grad"], ref["dJ"], floor=1e-6) <= 1e-7
+    ctx.close()
+
+
+@pytest.mark.parametrize("steps", [2, 5])
+@pytest.mark.parametrize("n", [24, 32, 40])   # first level 845, 1445 (of 2048) and, above the next, 2205 DOFs
+def test_coarse_levels_plate(oracle, mastg, n, steps):
+    """At rtol 1e-9: double precision does not reach 1e-10 on the larger plates
+    whatever the preconditioner, so the usual bars scale by ten with it."""
+    print(f"[coarse levels] plate {n}^2 steps {steps}", flush=True)
+    P = oracle.Problem(oracle.PLATE, n, n, seed=4)
+    ref = P.solve_elastic(1e-10)
+    ctx = ctx_from_oracle(mastg, P)
+    ctx.set_option(mastg.OPT_MG_STEPS_COARSE, steps)
+    r = ctx.design_eval(P.params(), rtol=1e-9, solver=mastg.SOLVER_MG)
+    assert r["rel_res"] <= 1.5e-9 and r["iters"] * 4 < ref["iters"], (r["iters"], ref["iters"])
+    assert abs(r["objective"] - ref["compliance"]) <= 1e-8 * abs(ref["compliance"])
+    assert rel_err_floor(r["grad"], ref["dc"], floor=1e-6) <= 1e-6
     ctx.close()
