@@ -1151,8 +1151,9 @@ bool lattice_args(mastg_ctx* c, CGArgs& a) {
 // one V-cycle on the problem-level vector r0 (null: the level-0 args' r); the
 // level-0 output is x0 + dlast0 (formed by the caller): returns dlast0.  The
 // matrix-free hex8 problem level (FP32) returns the output itself, with the
-// partial sums of r . output in a.part0 (started: the caller has written its
-// pre-smoothing start; the convergence test then runs beside the first pass)
+// partial sums of r . output in a.part0.  started: within a CG iteration, whose
+// convergence test then runs beside the first kernel (and whose update has
+// written the FP32 level's pre-smoothing start)
 const void* mg_vcycle(mastg_ctx* c, const CGArgs& a, const int* done, hipStream_t s, const double* r0 = nullptr,
                       bool started = false) {
     const int nl = int(c->mg.size());
@@ -1160,11 +1161,13 @@ const void* mg_vcycle(mastg_ctx* c, const CGArgs& a, const int* done, hipStream_
     MGLevelArgs L0 = D0.a;
     if (r0) L0.r = const_cast<double*>(r0);
     const bool f32 = L0.planar != 0;
+    const double* src0 = nullptr;
+    const int32_t* map0 = L0.rank_of_lat;
     if (D0.lat0) {
         // heat and hex8 on cells of several shapes: the problem level runs in
-        // lattice order (its output is mapped back to rank order by the
-        // caller: mg_rz / mg_bicg_iteration)
-        launch_perm_rank_lat(L0.n_nodes, L0.nav, L0.rank_of_lat, L0.r, D0.b_lat.as<double>(), 1, done, s);
+        // lattice order, from its first kernel on (its output is mapped back
+        // to rank order by the caller: mg_rz / mg_bicg_iteration)
+        src0 = L0.r;
         L0.r = D0.b_lat.as<double>();
         L0.dinv = D0.dinv_lat.as<double>();
         L0.con = D0.con_lat.as<uint8_t>();
@@ -1212,9 +1215,10 @@ const void* mg_vcycle(mastg_ctx* c, const CGArgs& a, const int* done, hipStream_
     for (int l = 0; l + 1 < nl && l < lt; l++) {
         const int k = steps(l);
         // coarse levels start their pre-smoothing inside the restriction
-        if (l == 0 && !started) launch_mg_pre_init(lv(l), done, s);
+        const CGCheck check = started ? CGCheck{a.S, a.part1, a.nvec} : CGCheck{};
+        if (l == 0 && !(f32 && started)) launch_mg_pre_init(lv(l), src0, map0, check, done, s);
         if (l == 0 && f32) {
-            if (started) S0.check = CGCheck{a.S, a.part1, a.nvec};
+            S0.check = check;
             for (int i = 1; i < k; i++) fine(i, i == 1, false, false);
             fine(0, true, true, false);
         } else {
@@ -1258,43 +1262,37 @@ const void* mg_vcycle(mastg_ctx* c, const CGArgs& a, const int* done, hipStream_
 void mg_rz(mastg_ctx* c, const CGArgs& a, const void* dl, hipStream_t s) {
     const MGLevelDev& D0 = *c->mg[0];
     const MGLevelArgs& L0 = D0.a;
-    if (D0.lat0) {   // z = x0 + dlast back in rank order, then r.z
-        launch_mg_combine_rank(L0.n_nodes, L0.nav, L0.rank_of_lat, L0.x, static_cast<const double*>(dl), a.z,
-                               &a.S->done, s);
-        launch_pcg_rz(a, a.z, nullptr, s);
-    } else {
-        launch_pcg_rz(a, L0.x, static_cast<const double*>(dl), s);
-    }
+    if (D0.lat0) launch_pcg_rz_rank(a, L0.nav, L0.rank_of_lat, L0.x, static_cast<const double*>(dl), s);
+    else launch_pcg_rz(a, L0.x, static_cast<const double*>(dl), s);
 }
 
+// an iteration has no kernel for scalars alone: each kernel sums the partials of
+// the one before it
 void mg_pcg_iteration(mastg_ctx* c, const CGArgs& a, hipStream_t s) {
     const int* done = &a.S->done;
     const MGLevelArgs& L0 = c->mg[0]->a;
-    if (L0.planar) {   // the lattice solver: no kernel for scalars alone
+    if (L0.planar) {   // the lattice solver
         launch_lattice_apply(a, a.p, a.q, s);
         launch_pcg_update_lat(a, L0, s);   // also starts the level-0 smoothing
         const void* z = mg_vcycle(c, a, done, s, nullptr, true);
-        launch_pcg_p_lat(a, static_cast<const float*>(z), int(lattice_partials(a.lat)), 0, s);
+        launch_pcg_p(a, static_cast<const float*>(z), int(lattice_partials(a.lat)), 0, s);
         return;
     }
-    launch_cg_op_alpha(a, s);
+    launch_cg_op(a, s);
     launch_pcg_update(a, s);
-    mg_rz(c, a, mg_vcycle(c, a, done, s), s);
-    launch_pcg_beta(a, s);
-    launch_cg_p(a, s);
+    mg_rz(c, a, mg_vcycle(c, a, done, s, nullptr, true), s);
+    launch_pcg_p(a, a.z, a.nvec, 0, s);
 }
 
 // z = M r and p = z, from the residual in a.r (the start of PCG, and its restarts)
-int mg_pcg_begin(mastg_ctx* c, const CGArgs& a, hipStream_t s) {
+void mg_pcg_begin(mastg_ctx* c, const CGArgs& a, hipStream_t s) {
     const void* z = mg_vcycle(c, a, &a.S->done, s);
     if (c->mg[0]->a.planar) {
-        launch_pcg_p_lat(a, static_cast<const float*>(z), int(lattice_partials(a.lat)), 1, s);
-        return MASTG_OK;
+        launch_pcg_p(a, static_cast<const float*>(z), int(lattice_partials(a.lat)), 1, s);
+        return;
     }
     mg_rz(c, a, z, s);
-    launch_pcg_start2(a, s);
-    HIPC(c, hipMemcpyAsync(a.p, a.z, c->S.n_active * sizeof(double), hipMemcpyDeviceToDevice, s));
-    return MASTG_OK;
+    launch_pcg_p(a, a.z, a.nvec, 1, s);
 }
 
 int mg_solve(mastg_ctx* c, const double* b, const mastg_solve_opts* o, mastg_solve_stats* st) {
@@ -1331,7 +1329,7 @@ int mg_solve(mastg_ctx* c, const double* b, const mastg_solve_opts* o, mastg_sol
     launch_fill(S.n_active, 0.0, a.x, c->stream);
     HIPC(c, hipMemcpyAsync(a.r, bl, S.n_active * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
     launch_pcg_start(a, bl, rtol * rtol, max_it, c->stream);
-    TRY(mg_pcg_begin(c, a, c->stream));
+    mg_pcg_begin(c, a, c->stream);
     HIPC(c, hipMemcpyAsync(c->h_scal, a.S, sizeof(CGScalars), hipMemcpyDeviceToHost, c->stream));
     HIPC(c, hipStreamSynchronize(c->stream));
     int done = c->h_scal->done;
@@ -1369,7 +1367,7 @@ int mg_solve(mastg_ctx* c, const double* b, const mastg_solve_opts* o, mastg_sol
                 if (rr < 0.25 * best2) stalls = 0;
                 else if (++stalls >= 8) { done = 5; break; }
                 best2 = std::min(best2, rr);
-                TRY(mg_pcg_begin(c, a, c->stream));
+                mg_pcg_begin(c, a, c->stream);
             }
         }
     }
@@ -1502,14 +1500,17 @@ int bicg_solve(mastg_ctx* c, const double* b, const mastg_solve_opts* o, mastg_s
     hipGraphExec_t& ex = mg ? c->mg_bicg_exec : c->bicg_exec;
     int& ex_len = mg ? c->mg_bicg_exec_len : c->bicg_exec_len;
     bool& ex_T = mg ? c->mg_bicg_exec_T : c->bicg_exec_T;
-    auto iteration = [&]() {
-        if (mg) mg_bicg_iteration(c, a, c->stream);
-        else launch_bicg_iteration(a, c->stream);
+    auto run_chunk = [&]() {
+        for (int i = 0; i < chunk; i++) {
+            if (mg) mg_bicg_iteration(c, a, c->stream);
+            else launch_bicg_iteration(a, c->stream);
+        }
+        launch_bicg_check(a, c->stream);
     };
     if (c->use_graphs) {
         if (!ex || ex_len != chunk || ex_T != transpose) {
             TRY(capture_graph(c, &ex, [&]() {
-                for (int i = 0; i < chunk; i++) iteration();
+                run_chunk();
             }));
             ex_len = chunk;
             ex_T = transpose;
@@ -1519,7 +1520,7 @@ int bicg_solve(mastg_ctx* c, const double* b, const mastg_solve_opts* o, mastg_s
     for (int launched = 0; launched < max_it + chunk; launched += chunk) {
         if (c->use_graphs) HIPC(c, hipGraphLaunch(ex, c->stream));
         else
-            for (int i = 0; i < chunk; i++) iteration();
+            run_chunk();
         HIPC(c, hipMemcpyAsync(c->h_pin, a.S, sizeof(BiCGScalars), hipMemcpyDeviceToHost, c->stream));
         HIPC(c, hipStreamSynchronize(c->stream));
         std::memcpy(&hs, c->h_pin, sizeof(BiCGScalars));

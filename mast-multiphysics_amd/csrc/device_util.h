@@ -49,6 +49,37 @@ __device__ __forceinline__ double reduce_partials(const double* __restrict__ p, 
     return t;
 }
 
+// two arrays of partials at once (their loads and exchanges overlap)
+__device__ __forceinline__ double2 reduce_partials2(const double* __restrict__ p, const double* __restrict__ q, int n) {
+    __shared__ double red[8];
+    double a0 = 0.0, a1 = 0.0, b0 = 0.0, b1 = 0.0;
+    int i = threadIdx.x;
+    for (; i + 256 < n; i += 512) {
+        a0 += p[i];
+        a1 += p[i + 256];
+        b0 += q[i];
+        b1 += q[i + 256];
+    }
+    if (i < n) {
+        a0 += p[i];
+        b0 += q[i];
+    }
+    double a = a0 + a1, b = b0 + b1;
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) {
+        a += __shfl_xor(a, m, 64);
+        b += __shfl_xor(b, m, 64);
+    }
+    if ((threadIdx.x & 63) == 0) {
+        red[threadIdx.x >> 6] = a;
+        red[4 + (threadIdx.x >> 6)] = b;
+    }
+    __syncthreads();
+    const double2 t = {(red[0] + red[1]) + (red[2] + red[3]), (red[4] + red[5]) + (red[6] + red[7])};
+    __syncthreads();
+    return t;
+}
+
 // block-level max of non-negative values into partials[slot]
 __device__ __forceinline__ void block_max_store(double v, double* partials, int slot) {
     __shared__ double red[4];

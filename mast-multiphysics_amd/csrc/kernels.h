@@ -128,9 +128,10 @@ struct ScatterArgs {
 };
 
 struct CGScalars {
-    double rz, pq, rr, bb, alpha, beta, tol2;
-    int iter, max_it, done, pad;
-    double rz2[2];   // the lattice solver's r.z of iteration i in rz2[i & 1]
+    double rr, bb, tol2;
+    int iter, max_it, done;
+    int next;        // the iteration that the vector kernels of plain CG are in
+    double rz2[2];   // r.z of iteration i in rz2[i & 1]
 };
 
 // the convergence test of a CG iteration, done by one work-group beside other
@@ -236,7 +237,7 @@ struct CGArgs {
 
 // right-preconditioned BiCGStab + Jacobi on a scalar CSR (PETSc KSPBCGS role)
 struct BiCGScalars {
-    double rho, rho_old, alpha, omega, beta, rr, bb, tol2;
+    double rho, rho_old, alpha, omega, rr, bb, tol2;
     int iter, max_it, done, pad;
 };
 struct BiCGArgs {
@@ -252,6 +253,7 @@ struct BiCGArgs {
 };
 void launch_bicg_start(const BiCGArgs& a, const double* b, double tol2, int max_it, hipStream_t s);
 void launch_bicg_iteration(const BiCGArgs& a, hipStream_t s);
+void launch_bicg_check(const BiCGArgs& a, hipStream_t s);   // after the last of a chunk of iterations
 // the iteration in three parts (p and ph = dinv p | v = A ph, alpha, s and sh =
 // dinv s | t = A sh, x, r, check) so a preconditioner can replace ph and sh
 void launch_bicg_part(const BiCGArgs& a, int part, hipStream_t s);
@@ -396,7 +398,11 @@ int64_t mg_invert_work(int n);
 double* mg_invert_input(int n, double* A, double* W);
 void launch_mg_invert(int n, double* A, double* W, hipStream_t s);
 // V-cycle pieces; every kernel returns at once when *done != 0 (done may be null)
-void launch_mg_pre_init(const MGLevelArgs& L, const int* done, hipStream_t s);
+// the problem level's start; a level in lattice order takes its right side from
+// the rank-ordered src (null: L.r); with CG's convergence test when check.S
+// (not for planar levels)
+void launch_mg_pre_init(const MGLevelArgs& L, const double* src, const int32_t* rank_of_lat, const CGCheck& check,
+                        const int* done, hipStream_t s);
 // the FP16 row-scaled copy of a lattice-order 27-point stencil ([27][n])
 void launch_sten27_to_f16(int64_t n, const float* sten, uint16_t* sten16, float* srow, hipStream_t s);
 // the FP16 row-scaled copy of a node-block matrix (val16, rs16 as above)
@@ -496,26 +502,28 @@ int64_t mg_tail_entries(int dim, int nav, int64_t n_nodes);
 hipError_t mg_tail_prepare();
 void launch_mg_tail_entries(const MGLevelArgs& L, float* ent, hipStream_t s);
 void launch_mg_tail(MGTailArgs A, int nav, const int* done, hipStream_t s);
-// preconditioned CG around the V-cycle
+// preconditioned CG around the V-cycle: alpha = r.z / p.q from the operator's
+// partial sums, x, r and the partials of r.r; the convergence test follows in
+// the V-cycle's first kernel (CGCheck)
 void launch_pcg_update(const CGArgs& c, hipStream_t s);
-// the lattice solver's: alpha = r.z / p.q from the operator's partial sums, the
-// update, and the start of the FP32 problem level L's pre-smoothing; the
-// convergence test follows beside the first smoothing pass (CGCheck)
+// the lattice solver's: with the start of the FP32 problem level L's pre-smoothing
 void launch_pcg_update_lat(const CGArgs& c, const MGLevelArgs& L, hipStream_t s);
-// its direction: r.z from n partial sums in c.part0, p = z (first) or z + beta p
-void launch_pcg_p_lat(const CGArgs& c, const float* z, int n, int first, hipStream_t s);
+// the direction: r.z from n partial sums in c.part0, p = z (first) or z + beta p
+void launch_pcg_p(const CGArgs& c, const float* z, int n, int first, hipStream_t s);
+void launch_pcg_p(const CGArgs& c, const double* z, int n, int first, hipStream_t s);
+// z = x0 + dlast (a V-cycle's level-0 output) and the nvec partial sums of r.z;
+// _rank: x0 and dlast in lattice order
 void launch_pcg_rz(const CGArgs& c, const double* x0, const double* dlast, hipStream_t s);
+void launch_pcg_rz_rank(const CGArgs& c, int nav, const int32_t* rank_of_lat, const double* x0, const double* dlast,
+                        hipStream_t s);
 void launch_pcg_start(const CGArgs& c, const double* b, double tol2, int max_it, hipStream_t s);
-void launch_pcg_start2(const CGArgs& c, hipStream_t s);
 // r.r of the current r (a restart's true residual): done = 1 / 0 / 2 as it meets tol
 void launch_pcg_recheck(const CGArgs& c, hipStream_t s);
-void launch_pcg_beta(const CGArgs& c, hipStream_t s);
 // out = x0 + dlast (a V-cycle's level-0 output), skipped when *done
 void launch_mg_combine(int64_t n, const double* x0, const double* dlast, double* out, const int* done,
                        hipStream_t s);
 // pieces of the CG iteration shared with the preconditioned variant
 void launch_mf_elem(const CGArgs& c, const double* x, hipStream_t s);   // element phase only
-void launch_cg_op_alpha(const CGArgs& c, hipStream_t s);                // q = A p, p.q, alpha
-void launch_cg_p(const CGArgs& c, hipStream_t s);                       // p = z + beta p
+void launch_cg_op(const CGArgs& c, hipStream_t s);                      // q = A p, partials of p.q
 
 }  // namespace mastg

@@ -1120,21 +1120,25 @@ __global__ __launch_bounds__(256) void k_spmv_csr_dot(CGArgs C, const double* __
     if (want_dot) block_sum_store(dsum, C.part0, blockIdx.x);
 }
 
-// alpha = rz / pq
-__global__ __launch_bounds__(256) void k_cg_alpha(CGArgs C) {
-    if (C.S->done) return;
-    const double pq = reduce_partials(C.part0, C.nparts_op);
-    if (threadIdx.x == 0) {
-        C.S->pq = pq;
-        C.S->alpha = C.S->rz / pq;
-        if (!(pq > 0.0) || !isfinite(pq)) C.S->done = 3;   // breakdown / NaN
-    }
-}
+// The iteration's scalars have no kernels of their own: each work-group sums
+// the partials of the kernel before it (a few KB from L2, about 1 us) instead
+// of waiting for a launch that does (2.2-3.6 us and a graph node's gap; the
+// iteration on 25,392 hex8 cells 25.9 -> 23.4 us).  A scalar that a kernel
+// updates is never one that its work-groups read: `iter` moves in k_cg_p,
+// `next` in k_cg_update, and r.z of iteration i lives in rz2[i & 1].
 
-// x += a p ; r -= a q ; z = dinv r ; partials (r.z, r.r)
+// alpha = r.z / p.q; x += alpha p; r -= alpha q; z = dinv r; partials of r.r, r.z
 __global__ __launch_bounds__(256) void k_cg_update(CGArgs C) {
-    if (C.S->done) return;
-    const double a = C.S->alpha;
+    CGScalars* S = C.S;
+    if (S->done) return;
+    const double pq = reduce_partials(C.part0, C.nparts_op);
+    if (!(pq > 0.0) || !isfinite(pq)) {   // breakdown / NaN, the same in every work-group
+        if (blockIdx.x == 0 && threadIdx.x == 0) S->done = 3;
+        return;
+    }
+    const int it = S->iter;
+    const double a = S->rz2[it & 1] / pq;
+    if (blockIdx.x == 0 && threadIdx.x == 0) S->next = it + 1;
     double rz = 0.0, rr = 0.0;
     for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < C.n; i += int64_t(gridDim.x) * 256) {
         C.x[i] += a * C.p[i];
@@ -1145,32 +1149,28 @@ __global__ __launch_bounds__(256) void k_cg_update(CGArgs C) {
         rz += r * z;
         rr += r * r;
     }
-    block_sum_store(rz, C.part0, blockIdx.x);
-    __syncthreads();
     block_sum_store(rr, C.part1, blockIdx.x);
+    __syncthreads();
+    block_sum_store(rz, C.part1 + C.nvec, blockIdx.x);
 }
 
-// beta = rz_new / rz ; convergence on ||r||^2 <= tol2 * ||b||^2
-__global__ __launch_bounds__(256) void k_cg_beta(CGArgs C) {
-    if (C.S->done) return;
-    const double rz = reduce_partials(C.part0, C.nvec);
-    const double rr = reduce_partials(C.part1, C.nvec);
-    if (threadIdx.x == 0) {
-        CGScalars* S = C.S;
-        S->beta = rz / S->rz;
-        S->rz = rz;
-        S->rr = rr;
-        S->iter += 1;
-        if (!isfinite(rr)) S->done = 4;
-        else if (rr <= S->tol2 * S->bb) S->done = 1;
-        else if (S->iter >= S->max_it) S->done = 2;
-    }
-}
-
-// p = z + beta p
+// convergence on ||r||^2 <= tol2 * ||b||^2 (p stays then); beta = r.z / the
+// last r.z; p = z + beta p
 __global__ __launch_bounds__(256) void k_cg_p(CGArgs C) {
-    if (C.S->done) return;
-    const double b = C.S->beta;
+    CGScalars* S = C.S;
+    if (S->done) return;
+    const double2 sums = reduce_partials2(C.part1, C.part1 + C.nvec, C.nvec);
+    const double rr = sums.x, rz = sums.y;
+    const int it = S->next;
+    const int done = !isfinite(rr) ? 4 : rr <= S->tol2 * S->bb ? 1 : it >= S->max_it ? 2 : 0;
+    const double b = rz / S->rz2[(it + 1) & 1];
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        S->rr = rr;
+        S->rz2[it & 1] = rz;
+        S->iter = it;
+        if (done) S->done = done;
+    }
+    if (done) return;
     for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < C.n; i += int64_t(gridDim.x) * 256)
         C.p[i] = C.z[i] + b * C.p[i];
 }
@@ -1196,7 +1196,7 @@ __global__ __launch_bounds__(256) void k_cg_start_scalars(CGArgs C, double tol2,
     const double bb = reduce_partials(C.part1, C.nvec);
     if (threadIdx.x == 0) {
         CGScalars* S = C.S;
-        S->rz = rz;
+        S->rz2[0] = rz;
         S->bb = bb;
         S->rr = bb;
         S->iter = 0;
@@ -1229,7 +1229,7 @@ __global__ __launch_bounds__(256) void k_cg_replace_scalars(CGArgs C) {
     const double rr = reduce_partials(C.part1, C.nvec);
     if (threadIdx.x == 0) {
         CGScalars* S = C.S;
-        S->rz = rz;
+        S->rz2[S->iter & 1] = rz;
         S->rr = rr;
         if (!isfinite(rr)) S->done = 4;
         else if (rr <= S->tol2 * S->bb) S->done = 1;
@@ -1326,6 +1326,10 @@ __global__ __launch_bounds__(256) void k_spmv_csr_gen(BiCGArgs B, const double* 
     }
 }
 
+// The scalars are folded into the vector kernels as in CG: each work-group sums
+// the partials itself, and a kernel writes no scalar that its work-groups read
+// (k_bicg_p: rho; k_bicg_s: alpha, rho_old; k_bicg_xr: omega, iter).  Partials:
+// r.r after the operator's in part0, r0.r after the operator's in part1.
 __global__ __launch_bounds__(256) void k_bicg_start(BiCGArgs B, const double* __restrict__ b) {
     double bb = 0.0;
     for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < B.n; i += int64_t(gridDim.x) * 256) {
@@ -1333,11 +1337,13 @@ __global__ __launch_bounds__(256) void k_bicg_start(BiCGArgs B, const double* __
         B.x[i] = 0.0; B.r[i] = v; B.r0[i] = v; B.p[i] = 0.0; B.v[i] = 0.0;
         bb += v * v;
     }
-    block_sum_store(bb, B.part0, blockIdx.x);
+    block_sum_store(bb, B.part0 + B.nparts, blockIdx.x);
+    __syncthreads();
+    block_sum_store(bb, B.part1 + B.nparts, blockIdx.x);   // r0 = r
 }
 
 __global__ __launch_bounds__(256) void k_bicg_start_s(BiCGArgs B, double tol2, int max_it) {
-    const double bb = reduce_partials(B.part0, B.nvec);
+    const double bb = reduce_partials(B.part0 + B.nparts, B.nvec);
     if (threadIdx.x == 0) {
         BiCGScalars* S = B.S;
         S->bb = bb; S->rr = bb; S->rho_old = 1.0; S->alpha = 1.0; S->omega = 1.0;
@@ -1346,47 +1352,47 @@ __global__ __launch_bounds__(256) void k_bicg_start_s(BiCGArgs B, double tol2, i
     }
 }
 
-// partial r0.r
-__global__ __launch_bounds__(256) void k_bicg_rho(BiCGArgs B) {
-    if (B.S->done) return;
-    double d = 0.0;
-    for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < B.n; i += int64_t(gridDim.x) * 256)
-        d += B.r0[i] * B.r[i];
-    block_sum_store(d, B.part0, blockIdx.x);
+// the outcome of the iterations so far (0: go on), from r.r of the last one
+__device__ __forceinline__ int bicg_outcome(const BiCGScalars* S, double rr) {
+    if (S->iter == 0) return 0;
+    return !isfinite(rr) ? 4 : rr <= S->tol2 * S->bb ? 1 : S->omega == 0.0 ? 3 : S->iter >= S->max_it ? 2 : 0;
 }
 
-// rho, beta; p = r + beta (p - omega v); ph = dinv p  (every block reduces the
-// partials itself: deterministic, one launch less)
+// convergence; rho, beta; p = r + beta (p - omega v); ph = dinv p
 __global__ __launch_bounds__(256) void k_bicg_p(BiCGArgs B) {
-    if (B.S->done) return;
-    const double rho = reduce_partials(B.part0, B.nvec);
-    const double beta = (rho / B.S->rho_old) * (B.S->alpha / B.S->omega);
-    const double om = B.S->omega;
+    BiCGScalars* S = B.S;
+    if (S->done) return;
+    const double2 sums = reduce_partials2(B.part0 + B.nparts, B.part1 + B.nparts, B.nvec);
+    const double rr = sums.x, rho = sums.y;
+    const int done = bicg_outcome(S, rr);
+    const double om = S->omega;
+    const double beta = (rho / S->rho_old) * (S->alpha / om);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        S->rr = rr;
+        S->rho = rho;
+        if (done) S->done = done;
+    }
+    if (done) return;
     for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < B.n; i += int64_t(gridDim.x) * 256) {
         const double p = B.r[i] + beta * (B.p[i] - om * B.v[i]);
         B.p[i] = p;
         B.ph[i] = B.dinv[i] * p;
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        B.S->beta = beta;
-        B.S->rho = rho;
-    }
 }
 
-// alpha = rho / r0.v
-__global__ __launch_bounds__(256) void k_bicg_alpha(BiCGArgs B) {
-    if (B.S->done) return;
-    const double r0v = reduce_partials(B.part0, B.nparts);
-    if (threadIdx.x == 0) {
-        B.S->alpha = B.S->rho / r0v;
-        if (!(r0v != 0.0) || !isfinite(r0v)) B.S->done = 3;
-    }
-}
-
-// s = r - alpha v ; sh = dinv s
+// alpha = rho / r0.v; s = r - alpha v ; sh = dinv s
 __global__ __launch_bounds__(256) void k_bicg_s(BiCGArgs B) {
-    if (B.S->done) return;
-    const double al = B.S->alpha;
+    BiCGScalars* S = B.S;
+    if (S->done) return;
+    const double r0v = reduce_partials(B.part0, B.nparts);
+    const bool bad = !(r0v != 0.0) || !isfinite(r0v);
+    const double rho = S->rho, al = rho / r0v;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        S->alpha = al;
+        S->rho_old = rho;
+        if (bad) S->done = 3;
+    }
+    if (bad) return;
     for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < B.n; i += int64_t(gridDim.x) * 256) {
         const double sv = B.r[i] - al * B.v[i];
         B.s[i] = sv;
@@ -1394,37 +1400,39 @@ __global__ __launch_bounds__(256) void k_bicg_s(BiCGArgs B) {
     }
 }
 
-// omega = (t.s)/(t.t); x += alpha ph + omega sh; r = s - omega t; partial r.r
+// omega = (t.s)/(t.t); x += alpha ph + omega sh; r = s - omega t; partials of
+// r.r and r0.r
 __global__ __launch_bounds__(256) void k_bicg_xr(BiCGArgs B) {
     if (B.S->done) return;
-    const double ts = reduce_partials(B.part0, B.nparts);
-    const double tt = reduce_partials(B.part1, B.nparts);
+    const double2 sums = reduce_partials2(B.part0, B.part1, B.nparts);
+    const double ts = sums.x, tt = sums.y;
     const double om = tt > 0.0 ? ts / tt : 0.0;
     const double al = B.S->alpha;
-    double rr = 0.0;
+    double rr = 0.0, rho = 0.0;
     for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < B.n; i += int64_t(gridDim.x) * 256) {
         B.x[i] += al * B.ph[i] + om * B.sh[i];
         const double rv = B.s[i] - om * B.t[i];
         B.r[i] = rv;
         rr += rv * rv;
+        rho += B.r0[i] * rv;
     }
-    __syncthreads();
     block_sum_store(rr, B.part0 + B.nparts, blockIdx.x);
-    if (blockIdx.x == 0 && threadIdx.x == 0) B.S->omega = om;
+    __syncthreads();
+    block_sum_store(rho, B.part1 + B.nparts, blockIdx.x);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        B.S->omega = om;
+        B.S->iter += 1;
+    }
 }
 
+// the outcome after the last iteration of a chunk, for the host
 __global__ __launch_bounds__(256) void k_bicg_check(BiCGArgs B) {
     if (B.S->done) return;
     const double rr = reduce_partials(B.part0 + B.nparts, B.nvec);
     if (threadIdx.x == 0) {
-        BiCGScalars* S = B.S;
-        S->rr = rr;
-        S->iter += 1;
-        S->rho_old = S->rho;
-        if (!isfinite(rr)) S->done = 4;
-        else if (rr <= S->tol2 * S->bb) S->done = 1;
-        else if (S->omega == 0.0) S->done = 3;
-        else if (S->iter >= S->max_it) S->done = 2;
+        B.S->rr = rr;
+        const int done = bicg_outcome(B.S, rr);
+        if (done) B.S->done = done;
     }
 }
 
@@ -1596,17 +1604,17 @@ void launch_bicg_start(const BiCGArgs& a, const double* b, double tol2, int max_
 }
 void launch_bicg_part(const BiCGArgs& a, int part, hipStream_t s) {
     if (part == 0) {
-        hipLaunchKernelGGL(k_bicg_rho, dim3(a.nvec), dim3(256), 0, s, a);
         hipLaunchKernelGGL(k_bicg_p, dim3(a.nvec), dim3(256), 0, s, a);
     } else if (part == 1) {
         spmv_gen(a, a.ph, a.v, a.r0, 0, s);
-        hipLaunchKernelGGL(k_bicg_alpha, dim3(1), dim3(256), 0, s, a);
         hipLaunchKernelGGL(k_bicg_s, dim3(a.nvec), dim3(256), 0, s, a);
     } else {
         spmv_gen(a, a.sh, a.t, a.s, 1, s);
         hipLaunchKernelGGL(k_bicg_xr, dim3(a.nvec), dim3(256), 0, s, a);
-        hipLaunchKernelGGL(k_bicg_check, dim3(1), dim3(256), 0, s, a);
     }
+}
+void launch_bicg_check(const BiCGArgs& a, hipStream_t s) {
+    hipLaunchKernelGGL(k_bicg_check, dim3(1), dim3(256), 0, s, a);
 }
 void launch_bicg_iteration(const BiCGArgs& a, hipStream_t s) {
     for (int part = 0; part < 3; part++) launch_bicg_part(a, part, s);
@@ -1648,7 +1656,7 @@ void launch_mf_elem(const CGArgs& c, const double* x, hipStream_t s) {
     else
         hipLaunchKernelGGL(k_hex8_mf_elem<false>, dim3(ge), dim3(256), 0, s, c, x);
 }
-void launch_cg_op_alpha(const CGArgs& c, hipStream_t s) {
+void launch_cg_op(const CGArgs& c, hipStream_t s) {
     if (c.use_mf == 1)
         mf_dispatch(c, c.p, c.p, c.q, 1, s);
     else if (c.use_mf == 2)
@@ -1657,21 +1665,10 @@ void launch_cg_op_alpha(const CGArgs& c, hipStream_t s) {
         nb64_dispatch(c, c.p, c.q, 1, 1, s);
     else
         spmv_dispatch(c, c.p, c.q, 1, 1, s);
-    hipLaunchKernelGGL(k_cg_alpha, dim3(1), dim3(256), 0, s, c);
-}
-void launch_cg_p(const CGArgs& c, hipStream_t s) {
-    hipLaunchKernelGGL(k_cg_p, dim3(c.nvec), dim3(256), 0, s, c);
 }
 void launch_cg_iteration(const CGArgs& c, hipStream_t s) {
-    if (c.use_mf == 1)
-        mf_dispatch(c, c.p, c.p, c.q, 1, s);
-    else if (c.use_mf == 2)
-        nb32_dispatch(c, c.p, c.q, 1, 1, s);
-    else
-        spmv_dispatch(c, c.p, c.q, 1, 1, s);
-    hipLaunchKernelGGL(k_cg_alpha, dim3(1), dim3(256), 0, s, c);
+    launch_cg_op(c, s);
     hipLaunchKernelGGL(k_cg_update, dim3(c.nvec), dim3(256), 0, s, c);
-    hipLaunchKernelGGL(k_cg_beta, dim3(1), dim3(256), 0, s, c);
     hipLaunchKernelGGL(k_cg_p, dim3(c.nvec), dim3(256), 0, s, c);
 }
 

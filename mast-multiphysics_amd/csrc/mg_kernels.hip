@@ -205,11 +205,29 @@ __device__ __forceinline__ void mg_epilogue(const MGLevelArgs& L, int mode, int6
     }
 }
 
-__global__ __launch_bounds__(256) void k_mg_pre_init(MGLevelArgs L, const int* __restrict__ done) {
+// The start of the problem level's pre-smoothing (x = 0, res = r, the first
+// direction), with two neighbours' work in the same launch: a level in lattice
+// order takes r from the rank-ordered vector src (null: L.r itself) and writes
+// it to L.r, and the last work-group makes CG's convergence test (check).
+__global__ __launch_bounds__(256) void k_mg_pre_init(MGLevelArgs L, const double* __restrict__ src,
+                                                     const int32_t* __restrict__ rank_of_lat, CGCheck check,
+                                                     const int* __restrict__ done) {
     if (done && *done) return;
+    const int64_t nb = gridDim.x - (check.S ? 1 : 0);
+    if (int64_t(blockIdx.x) == nb) {
+        pcg_check_block(check);
+        return;
+    }
     const double ith = L.cheb[0];
-    for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < L.n_nodes * L.nav; i += int64_t(gridDim.x) * 256) {
-        const double r = L.r[i];
+    for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < L.n_nodes * L.nav; i += nb * 256) {
+        double r;
+        if (src) {
+            const int64_t p = i / L.nav;
+            r = src[int64_t(rank_of_lat[p]) * L.nav + (i - p * L.nav)];
+            L.r[i] = r;
+        } else {
+            r = L.r[i];
+        }
         L.x[i] = 0.0;
         L.res[i] = r;
         L.da[i] = L.dinv[i] * r * ith;
@@ -219,10 +237,15 @@ __global__ __launch_bounds__(256) void k_mg_pre_init(MGLevelArgs L, const int* _
 // the same start with block Jacobi (5 variables per node): da = ith Dinv_b r,
 // a thread per DOF (row v of node n's inverse block), so that a wave's loads
 // of the blocks and of r cover contiguous memory
-__global__ __launch_bounds__(256) void k_mg_pre_init_blk5(MGLevelArgs L, const int* __restrict__ done) {
+__global__ __launch_bounds__(256) void k_mg_pre_init_blk5(MGLevelArgs L, CGCheck check, const int* __restrict__ done) {
     if (done && *done) return;
+    const int64_t nb = gridDim.x - (check.S ? 1 : 0);
+    if (int64_t(blockIdx.x) == nb) {
+        pcg_check_block(check);
+        return;
+    }
     const double ith = L.cheb[0];
-    for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < L.n_nodes * 5; i += int64_t(gridDim.x) * 256) {
+    for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < L.n_nodes * 5; i += nb * 256) {
         const int64_t n = i / 5;
         const double* rn = L.r + n * 5;
         const float* B = L.dinvb + i * 5;   // row v = i - 5 n of node n's block
@@ -1260,11 +1283,25 @@ __global__ __launch_bounds__(256) void k_mg_coarse_solve(int n, const double* __
 }
 
 // ---- preconditioned CG ---------------------------------------------------------
+// alpha = r.z / p.q, p.q from the operator's partials, summed by every
+// work-group (a launch less than a kernel for alpha); false: breakdown / NaN,
+// the same in every work-group
+__device__ __forceinline__ bool pcg_alpha(const CGArgs& C, double& a) {
+    CGScalars* S = C.S;
+    const double pq = reduce_partials(C.part0, C.nparts_op);
+    if (!(pq > 0.0) || !isfinite(pq)) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) S->done = 3;
+        return false;
+    }
+    a = S->rz2[S->iter & 1] / pq;
+    return true;
+}
+
 // x += alpha p ; r -= alpha q ; partials r.r
 __global__ __launch_bounds__(256) void k_pcg_update(CGArgs C) {
     if (C.S->done) return;
-    const double a = C.S->alpha;
-    double rr = 0.0;
+    double a, rr = 0.0;
+    if (!pcg_alpha(C, a)) return;
     for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < C.n; i += int64_t(gridDim.x) * 256) {
         C.x[i] += a * C.p[i];
         const double r = C.r[i] - a * C.q[i];
@@ -1274,20 +1311,13 @@ __global__ __launch_bounds__(256) void k_pcg_update(CGArgs C) {
     block_sum_store(rr, C.part1, blockIdx.x);
 }
 
-// the lattice solver's update: every work-group sums the operator's partials
-// of p.q itself (a launch less than a kernel for alpha); x, r, the partials of
-// r.r, and the start of the FP32 pre-smoothing (b = r, x = D^-1 b / theta)
+// the lattice solver's update: x, r, the partials of r.r, and the start of the
+// FP32 pre-smoothing (b = r, x = D^-1 b / theta)
 __global__ __launch_bounds__(256) void k_pcg_update_lat(CGArgs C, MGLevelArgs L) {
-    CGScalars* S = C.S;
-    if (S->done) return;
-    const double pq = reduce_partials(C.part0, C.nparts_op);
-    if (!(pq > 0.0) || !isfinite(pq)) {   // breakdown / NaN, the same in every work-group
-        if (blockIdx.x == 0 && threadIdx.x == 0) S->done = 3;
-        return;
-    }
-    const double a = S->rz2[S->iter & 1] / pq;
+    if (C.S->done) return;
+    double a, rr = 0.0;
+    if (!pcg_alpha(C, a)) return;
     const float ith = float(L.cheb[0]);
-    double rr = 0.0;
     for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < C.n; i += int64_t(gridDim.x) * 256) {
         C.x[i] += a * C.p[i];
         const double r = C.r[i] - a * C.q[i];
@@ -1302,7 +1332,8 @@ __global__ __launch_bounds__(256) void k_pcg_update_lat(CGArgs C, MGLevelArgs L)
 
 // r.z summed by every work-group, beta = r.z / the last r.z, p = z + beta p
 // (first: p = z); a non-positive r.z means the preconditioner is not SPD
-__global__ __launch_bounds__(256) void k_pcg_p_lat(CGArgs C, const float* __restrict__ z, int n, int first) {
+template <typename T>
+__global__ __launch_bounds__(256) void k_pcg_p(CGArgs C, const T* __restrict__ z, int n, int first) {
     CGScalars* S = C.S;
     if (S->done) return;
     const double rz = reduce_partials(C.part0, n);
@@ -1315,12 +1346,6 @@ __global__ __launch_bounds__(256) void k_pcg_p_lat(CGArgs C, const float* __rest
     if (blockIdx.x == 0 && threadIdx.x == 0) S->rz2[it & 1] = rz;
     for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < C.n; i += int64_t(gridDim.x) * 256)
         C.p[i] = first ? double(z[i]) : double(z[i]) + beta * C.p[i];
-}
-
-// convergence on the updated residual, before the V-cycle runs
-__global__ __launch_bounds__(256) void k_pcg_check(CGArgs C) {
-    if (C.S->done) return;
-    pcg_check_block(CGCheck{C.S, C.part1, C.nvec});
 }
 
 // z = x0 + dlast (the level-0 V-cycle output) ; partials r.z
@@ -1336,24 +1361,27 @@ __global__ __launch_bounds__(256) void k_pcg_rz(CGArgs C, const double* __restri
     block_sum_store(rz, C.part0, blockIdx.x);
 }
 
-// beta = rz_new / rz ; a non-positive r.z means the preconditioner is not SPD
+// the same for a problem level in lattice order: z and r in rank order
+__global__ __launch_bounds__(256) void k_pcg_rz_rank(CGArgs C, int nav, const int32_t* __restrict__ rank_of_lat,
+                                                     const double* __restrict__ x0,
+                                                     const double* __restrict__ dlast) {
+    if (C.S->done) return;
+    double rz = 0.0;
+    for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < C.n; i += int64_t(gridDim.x) * 256) {
+        const int64_t p = i / nav, k = int64_t(rank_of_lat[p]) * nav + (i - p * nav);
+        const double z = x0[i] + dlast[i];
+        C.z[k] = z;
+        rz += C.r[k] * z;
+    }
+    block_sum_store(rz, C.part0, blockIdx.x);
+}
+
 __global__ __launch_bounds__(256) void k_mg_combine(int64_t n, const double* __restrict__ x0,
                                                     const double* __restrict__ dlast, double* __restrict__ out,
                                                     const int* __restrict__ done) {
     if (done && *done) return;
     for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < n; i += int64_t(gridDim.x) * 256)
         out[i] = dlast ? x0[i] + dlast[i] : x0[i];
-}
-
-__global__ __launch_bounds__(256) void k_pcg_beta(CGArgs C) {
-    if (C.S->done) return;
-    const double rz = reduce_partials(C.part0, C.nvec);
-    if (threadIdx.x == 0) {
-        CGScalars* S = C.S;
-        if (!(rz > 0.0) || !isfinite(rz)) { S->done = 3; return; }
-        S->beta = rz / S->rz;
-        S->rz = rz;
-    }
 }
 
 __global__ __launch_bounds__(256) void k_pcg_start(CGArgs C, const double* __restrict__ b) {
@@ -1369,7 +1397,6 @@ __global__ __launch_bounds__(256) void k_pcg_start_scalars(CGArgs C, double tol2
         CGScalars* S = C.S;
         S->bb = bb;
         S->rr = bb;
-        S->rz = 0.0;
         S->iter = 0;
         S->tol2 = tol2;
         S->max_it = max_it;
@@ -1387,15 +1414,6 @@ __global__ __launch_bounds__(256) void k_pcg_recheck(CGArgs C) {
         else if (rr <= S->tol2 * S->bb) S->done = 1;
         else if (S->iter >= S->max_it) S->done = 2;
         else S->done = 0;
-    }
-}
-
-__global__ __launch_bounds__(256) void k_pcg_start2(CGArgs C) {
-    if (C.S->done) return;
-    const double rz = reduce_partials(C.part0, C.nvec);
-    if (threadIdx.x == 0) {
-        if (!(rz > 0.0) || !isfinite(rz)) C.S->done = 3;
-        C.S->rz = rz;
     }
 }
 
@@ -1496,10 +1514,12 @@ void launch_perm_nodes(int64_t n_nodes, const int32_t* map, const double* src, d
                        hipStream_t s) {
     hipLaunchKernelGGL(k_perm_nodes, dim3(mg_blocks(n_nodes, 256)), dim3(256), 0, s, n_nodes, map, src, dst, scatter);
 }
-void launch_mg_pre_init(const MGLevelArgs& L, const int* done, hipStream_t s) {
+void launch_mg_pre_init(const MGLevelArgs& L, const double* src, const int32_t* rank_of_lat, const CGCheck& check,
+                        const int* done, hipStream_t s) {
+    const dim3 g(mg_grid(L.n_nodes * L.nav) + (check.S ? 1 : 0));
     if (L.planar) hipLaunchKernelGGL(k_mg_pre_init32, dim3(mg_grid(L.n_nodes * L.nav)), dim3(256), 0, s, L, done);
-    else if (L.dinvb) hipLaunchKernelGGL(k_mg_pre_init_blk5, dim3(mg_grid(L.n_nodes * 5)), dim3(256), 0, s, L, done);
-    else hipLaunchKernelGGL(k_mg_pre_init, dim3(mg_grid(L.n_nodes * L.nav)), dim3(256), 0, s, L, done);
+    else if (L.dinvb) hipLaunchKernelGGL(k_mg_pre_init_blk5, g, dim3(256), 0, s, L, check, done);
+    else hipLaunchKernelGGL(k_mg_pre_init, g, dim3(256), 0, s, L, src, rank_of_lat, check, done);
 }
 void launch_mg_block_dinv5(const MGLevelArgs& L, float* dinvb, hipStream_t s) {
     hipLaunchKernelGGL(k_mg_block_dinv5, dim3(mg_blocks(L.n_nodes, 256)), dim3(256), 0, s, L, dinvb);
@@ -1615,23 +1635,26 @@ void launch_mg_coarse_solve(int n, const double* Ainv, const double* r, double* 
 }
 void launch_pcg_update(const CGArgs& c, hipStream_t s) {
     hipLaunchKernelGGL(k_pcg_update, dim3(c.nvec), dim3(256), 0, s, c);
-    hipLaunchKernelGGL(k_pcg_check, dim3(1), dim3(256), 0, s, c);
 }
 void launch_pcg_update_lat(const CGArgs& c, const MGLevelArgs& L, hipStream_t s) {
     hipLaunchKernelGGL(k_pcg_update_lat, dim3(c.nvec), dim3(256), 0, s, c, L);
 }
-void launch_pcg_p_lat(const CGArgs& c, const float* z, int n, int first, hipStream_t s) {
-    hipLaunchKernelGGL(k_pcg_p_lat, dim3(c.nvec), dim3(256), 0, s, c, z, n, first);
+void launch_pcg_p(const CGArgs& c, const float* z, int n, int first, hipStream_t s) {
+    hipLaunchKernelGGL(k_pcg_p<float>, dim3(c.nvec), dim3(256), 0, s, c, z, n, first);
+}
+void launch_pcg_p(const CGArgs& c, const double* z, int n, int first, hipStream_t s) {
+    hipLaunchKernelGGL(k_pcg_p<double>, dim3(c.nvec), dim3(256), 0, s, c, z, n, first);
 }
 void launch_pcg_rz(const CGArgs& c, const double* x0, const double* dlast, hipStream_t s) {
     hipLaunchKernelGGL(k_pcg_rz, dim3(c.nvec), dim3(256), 0, s, c, x0, dlast);
 }
+void launch_pcg_rz_rank(const CGArgs& c, int nav, const int32_t* rank_of_lat, const double* x0, const double* dlast,
+                        hipStream_t s) {
+    hipLaunchKernelGGL(k_pcg_rz_rank, dim3(c.nvec), dim3(256), 0, s, c, nav, rank_of_lat, x0, dlast);
+}
 void launch_mg_combine(int64_t n, const double* x0, const double* dlast, double* out, const int* done,
                        hipStream_t s) {
     hipLaunchKernelGGL(k_mg_combine, dim3(mg_grid(n)), dim3(256), 0, s, n, x0, dlast, out, done);
-}
-void launch_pcg_beta(const CGArgs& c, hipStream_t s) {
-    hipLaunchKernelGGL(k_pcg_beta, dim3(1), dim3(256), 0, s, c);
 }
 void launch_pcg_start(const CGArgs& c, const double* b, double tol2, int max_it, hipStream_t s) {
     hipLaunchKernelGGL(k_pcg_start, dim3(c.nvec), dim3(256), 0, s, c, b);
@@ -1640,9 +1663,6 @@ void launch_pcg_start(const CGArgs& c, const double* b, double tol2, int max_it,
 void launch_pcg_recheck(const CGArgs& c, hipStream_t s) {
     hipLaunchKernelGGL(k_pcg_start, dim3(c.nvec), dim3(256), 0, s, c, c.r);
     hipLaunchKernelGGL(k_pcg_recheck, dim3(1), dim3(256), 0, s, c);
-}
-void launch_pcg_start2(const CGArgs& c, hipStream_t s) {
-    hipLaunchKernelGGL(k_pcg_start2, dim3(1), dim3(256), 0, s, c);
 }
 
 }  // namespace mastg
