@@ -223,7 +223,8 @@ struct CGArgs {
     int nvec;                 // grid of the CG vector kernels (and their partials)
     CGScalars* S;
     int use_mf;               // operator: 0 CSR SpMV, 1 matrix-free, 2 FP32 node-block SpMV,
-                              // 3 hex8 lattice operator (PCG only), 4 FP64 node-block SpMV
+                              // 3 hex8 lattice operator (vectors in lattice order), 4 FP64
+                              // node-block SpMV (PCG only)
     int spmv_sw;              // CSR SpMV lanes per row (4, 8, 16, 32, 64)
     MFArgs mf;
     // FP32 copy of the CSR values read by node blocks (operator 2): node rank

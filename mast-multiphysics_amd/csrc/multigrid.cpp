@@ -160,6 +160,11 @@ bool detect_lattice_topology(const Structure& S, int dim, MGLevelHost& L, std::s
 
 }  // namespace
 
+bool find_box_lattice(const Structure& S, MGLevelHost& L) {
+    std::string why;
+    return S.nav == 3 && S.npe == 8 && detect_lattice(S, 3, L, why);
+}
+
 MGHierarchy build_mg_hierarchy(const Structure& S) {
     MGHierarchy H;
     int dim = 0, physics = 0;

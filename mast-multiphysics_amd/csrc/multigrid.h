@@ -47,6 +47,10 @@ constexpr int64_t kMGCoarseTarget = 136;
 // Detects the lattice and builds the coarse levels (hex8: nav 3, quad4: nav 5).
 MGHierarchy build_mg_hierarchy(const Structure& S);
 
+// The lattice of a mesh of equal axis-aligned boxes (no coarse levels; any cell
+// counts); false when the mesh is none.
+bool find_box_lattice(const Structure& S, MGLevelHost& L);
+
 // One-class hex8 lattice: Gc[c] = Q_c^T Khat Q_c ([8][64 blocks][3x3], block
 // (A, B) at (A 8 + B) 9) for the 8 children c of a coarse cell, made exactly
 // symmetric.  Khat: [64][3x3] in the same layout.

@@ -75,3 +75,39 @@ def test_box_smoothing_steps(oracle, mastg, steps):
         assert abs(r["objective"] - ref["compliance"]) <= 1e-9 * abs(ref["compliance"])
         assert rel_err_floor(r["grad"], ref["dc"], floor=1e-6) <= 1e-7
     ctx.close()
+
+
+# lattices that do not coarsen, down to one cell; rows of 62 and 63 points (a
+# wave's share and one over); nodes and elements as the mesh generator numbers
+# them and shuffled
+@pytest.mark.parametrize("shuffle", [False, True])
+@pytest.mark.parametrize("mesh", [(1, 1, 1), (3, 1, 1), (2, 3, 1), (7, 9, 11), (61, 2, 2), (62, 3, 1), (45, 23, 23)])
+def test_matrix_free_cg_equals_csr_cg(oracle, mastg, mesh, shuffle):
+    """Matrix-free CG on equal boxes runs the lattice product with its vectors
+    in lattice order: the same Krylov iteration as on the assembled CSR, and
+    the same answers."""
+    print(f"[matrix-free CG] {mesh} shuffle={shuffle}", flush=True)
+    P = oracle.Problem(oracle.CANTILEVER, *mesh, seed=4, lo=0.1, hi=1.0)
+    xyz, conn = P.mesh()
+    base, con = P.dofmap()
+    rng = np.random.default_rng(11)
+    if shuffle:
+        node = rng.permutation(len(xyz))            # new node of each old one
+        elem = rng.permutation(len(conn))
+        xyz2, base2 = np.empty_like(xyz), np.empty_like(base)
+        xyz2[node], base2[node] = xyz, base
+        xyz, base, conn = xyz2, base2, node[conn][elem].astype(conn.dtype)
+    desc = mastg.desc_from_arrays(mastg.HEX8_ELASTIC, xyz, conn, P.n_vars, node_dof_base=base,
+                                  constrained_dofs=np.nonzero(con)[0], point_loads=P.point_load(), E=72e9, nu=0.33,
+                                  penalty=3.0)
+    ctx = mastg.Context(desc)
+    ctx._keep = desc
+    rho = rng.uniform(0.1, 1.0, len(conn))
+    ref = ctx.design_eval(rho)
+    for _ in range(2):                               # the first solve finds the lattice
+        r = ctx.design_eval(rho, solver=mastg.SOLVER_MATFREE)
+        assert r["rel_res"] <= 1.5e-10
+        assert abs(r["iters"] - ref["iters"]) <= 2 + ref["iters"] // 50, (r["iters"], ref["iters"])
+        assert abs(r["objective"] - ref["objective"]) <= 1e-9 * abs(ref["objective"])
+        assert rel_err_floor(r["grad"], ref["grad"], floor=1e-6) <= 1e-7
+    ctx.close()
