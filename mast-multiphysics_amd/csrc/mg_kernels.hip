@@ -441,56 +441,130 @@ __global__ __launch_bounds__(256) void k_mg_to_stencil(MGLevelArgs L, float* __r
     }
 }
 
-// Smoothing step of a stencil level: thread per node, coalesced FP32 stencil
-// loads, FP64 products and sums, the fused Chebyshev epilogue
-__global__ __launch_bounds__(256) void k_mg_stencil(MGLevelArgs L, const float* __restrict__ sten, int mode, int step,
-                                                    const double* __restrict__ din, double* __restrict__ dout,
-                                                    const int* __restrict__ done) {
+// Smoothing step of a stencil level: 64 nodes per work-group, a wave per z-layer
+// of offsets, the three layers' sums exchanged through LDS, then a thread per
+// DOF for the fused Chebyshev epilogue.  FP32 stencil, FP64 products and sums.
+// A wave's neighbours towards (dy, dz) are 66 consecutive nodes: their vector
+// goes through LDS (a lane's own loads, 24 bytes apart and three for every row,
+// kept the address units busy), the stencil by coalesced buffer loads, a row of
+// 27 entries at a time (two or three rows at once take the registers of a wave
+// or two per SIMD: 11.2 us at 65x33x33 nodes).  What lies outside the arrays
+// reads as 0.  There a thread per node took 16.4 us (one wave per SIMD), a wave
+// per layer with its own vector loads 12.8, from LDS 10.4: 500 B of stencil per
+// node, each read twice, at 6.5 TB/s.  At 33x17x17, bound by latency, 4.7 us.
+constexpr int kStenNodes = 64;
+constexpr int kStenRun = 3 * (kStenNodes + 2);   // doubles of a row's vector
+
+typedef uint32_t sten_u2 __attribute__((ext_vector_type(2)));
+
+template <int LZ>
+__device__ __forceinline__ void stencil_layer(const MGLevelArgs& L, const float* __restrict__ sten,
+                                              const double* __restrict__ in, uint32_t r0, double (&xs)[3][kStenRun],
+                                              double (&y)[3]) {
+    const uint32_t N = uint32_t(L.n_nodes), nxp = uint32_t(L.nx + 1), nyp = uint32_t(L.ny + 1);
+    const uint32_t lane = threadIdx.x & (kStenNodes - 1), r = r0 + lane, rq = r / nxp;
+    const int i = int(r - rq * nxp), j = int(rq % nyp), k = int(rq / nyp);
+    // row dy of the layer, offset dx: the 9 entries (3 v + w) of the block
+    // towards r + off: r's own (o - 14) 9 + 3 v + w, or the neighbour's
+    // (12 - o) 9 + 3 w + v for o < 13, or r's 6 symmetric ones for o = 13
+    auto entries = [&](int row, float (&e)[27]) {
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            const int o = LZ * 9 + row * 3 + d;
+            const int off = (d - 1) + int(nxp) * ((row - 1) + int(nyp) * (LZ - 1));
+            const int e0 = o == 13 ? 117 : o < 13 ? (12 - o) * 9 : (o - 14) * 9;
+            const auto rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(sten + int64_t(e0) * N), 0,
+                                                              (o == 13 ? 6 : 9) * N * 4u, 0x00020000);
+            const uint32_t at = (r + uint32_t(o < 13 ? off : 0)) * 4u;
+#pragma unroll
+            for (int q = 0; q < 9; q++) {
+                const int v = q / 3, w = q % 3;
+                const int f = o == 13 ? (v <= w ? v * (5 - v) / 2 + w : w * (5 - w) / 2 + v) : o < 13 ? 3 * w + v : q;
+                if (o == 13 && v > w) continue;   // the same as (w, v)
+                e[d * 9 + q] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, at, f * N * 4u, 0));
+            }
+            if (o == 13) {
+                e[d * 9 + 3] = e[d * 9 + 1];
+                e[d * 9 + 6] = e[d * 9 + 2];
+                e[d * 9 + 7] = e[d * 9 + 5];
+            }
+        }
+    };
+    const auto xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<double*>(in), 0, N * 24u, 0x00020000);
+    constexpr int NT = (kStenRun + kStenNodes - 1) / kStenNodes;
+    sten_u2 q[3][NT];
+#pragma unroll
+    for (int row = 0; row < 3; row++) {
+        const uint32_t first = (r0 + uint32_t(int(nxp) * ((row - 1) + int(nyp) * (LZ - 1)) - 1)) * 24u;
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+            q[row][t] = __builtin_amdgcn_raw_buffer_load_b64(xr, first + (t * kStenNodes + lane) * 8u, 0, 0);
+    }
+    // loads return in the order of issue: the vector's first
+    __builtin_amdgcn_sched_barrier(0);
+    float e[27];
+    entries(0, e);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int row = 0; row < 3; row++)
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+            if (t * kStenNodes + lane < kStenRun)
+                xs[row][t * kStenNodes + lane] = __longlong_as_double((long long)(uint64_t(q[row][t][1]) << 32 | q[row][t][0]));
+    __syncthreads();
+    double y0 = 0.0, y1 = 0.0, y2 = 0.0;
+#pragma unroll
+    for (int row = 0; row < 3; row++) {
+        if (row > 0) entries(row, e);
+        const bool in_yz = j + row >= 1 && j + row <= L.ny + 1 && k + LZ >= 1 && k + LZ <= L.nz + 1;
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            const int o = LZ * 9 + row * 3 + d;
+            double x0 = xs[row][3 * (lane + d)], x1 = xs[row][3 * (lane + d) + 1], x2 = xs[row][3 * (lane + d) + 2];
+            if (o < 13) {   // a neighbour outside the lattice (its own entries there are 0)
+                const bool inside = in_yz && i + d >= 1 && i + d <= L.nx + 1;
+                x0 = inside ? x0 : 0.0;
+                x1 = inside ? x1 : 0.0;
+                x2 = inside ? x2 : 0.0;
+            }
+            const float* q = &e[d * 9];
+            y0 = fma(double(q[2]), x2, fma(double(q[1]), x1, fma(double(q[0]), x0, y0)));
+            y1 = fma(double(q[5]), x2, fma(double(q[4]), x1, fma(double(q[3]), x0, y1)));
+            y2 = fma(double(q[8]), x2, fma(double(q[7]), x1, fma(double(q[6]), x0, y2)));
+        }
+    }
+    y[0] = y0;
+    y[1] = y1;
+    y[2] = y2;
+}
+
+__global__ __launch_bounds__(3 * kStenNodes) void k_mg_stencil(MGLevelArgs L, const float* __restrict__ sten, int mode,
+                                                               int step, const double* __restrict__ din,
+                                                               double* __restrict__ dout,
+                                                               const int* __restrict__ done) {
     if (done && *done) return;
+    __shared__ double xs[3][3][kStenRun];
     // work-groups in XCD-aware order: the neighbouring rows whose stored
     // blocks this row reads transposed were read by work-groups of the same
     // XCD (its L2), not of another
-    const int64_t r = xcd_block(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
-    if (r >= L.n_nodes) return;
-    const int64_t N = L.n_nodes;
+    const uint32_t r0 = uint32_t(xcd_block(blockIdx.x, gridDim.x)) * kStenNodes;
+    const int lane = threadIdx.x & (kStenNodes - 1), layer = __builtin_amdgcn_readfirstlane(threadIdx.x / kStenNodes);
     const double* __restrict__ in = mode == MG_RESID_INIT ? L.x : din;
-    const uint32_t nxp = uint32_t(L.nx + 1), nyp = uint32_t(L.ny + 1), ru = uint32_t(r), rq = ru / nxp;
-    const int i = int(ru - rq * nxp), j = int(rq % nyp), k = int(rq / nyp);
-    double y0, y1, y2;
-    {   // own block (symmetric)
-        const float* __restrict__ S = sten + 117 * N + r;
-        const double s00 = S[0], s01 = S[N], s02 = S[2 * N], s11 = S[3 * N], s12 = S[4 * N], s22 = S[5 * N];
-        const double x0 = in[r * 3], x1 = in[r * 3 + 1], x2 = in[r * 3 + 2];
-        y0 = fma(s02, x2, fma(s01, x1, s00 * x0));
-        y1 = fma(s12, x2, fma(s11, x1, s01 * x0));
-        y2 = fma(s22, x2, fma(s12, x1, s02 * x0));
-    }
-    // the 26 neighbours, one z-layer of 9 offsets per pass (bounded loads in flight)
-#pragma unroll 9
-    for (int o = 0; o < 27; o++) {
-        if (o == 13) continue;
-        const int ui = i + o % 3 - 1, uj = j + (o / 3) % 3 - 1, uk = k + o / 9 - 1;
-        const bool inside = ui >= 0 && ui <= L.nx && uj >= 0 && uj <= L.ny && uk >= 0 && uk <= L.nz;
-        const int ni = min(max(ui, 0), L.nx), nj = min(max(uj, 0), L.ny), nk = min(max(uk, 0), L.nz);
-        const int64_t m = int64_t(uint32_t(ni) + nxp * (uint32_t(nj) + nyp * uint32_t(nk)));
-        // a neighbour outside the lattice is clamped into it and weighted 0
-        const double wgt = inside ? 1.0 : 0.0;
-        const double x0 = wgt * in[m * 3], x1 = wgt * in[m * 3 + 1], x2 = wgt * in[m * 3 + 2];
-        // block (v, w) towards m: own entry (o - 14) 9 + 3 v + w at r, or the
-        // neighbour's entry (12 - o) 9 + 3 w + v at m (uniform strides)
-        const bool lower = o < 13;
-        const float* __restrict__ S = lower ? sten + int64_t(12 - o) * 9 * N + m : sten + int64_t(o - 14) * 9 * N + r;
-        const int64_t sv = lower ? N : 3 * N, sw = lower ? 3 * N : N;
-        y0 = fma(double(S[0]), x0, y0); y0 = fma(double(S[sw]), x1, y0); y0 = fma(double(S[2 * sw]), x2, y0);
-        y1 = fma(double(S[sv]), x0, y1); y1 = fma(double(S[sv + sw]), x1, y1); y1 = fma(double(S[sv + 2 * sw]), x2, y1);
-        y2 = fma(double(S[2 * sv]), x0, y2); y2 = fma(double(S[2 * sv + sw]), x1, y2);
-        y2 = fma(double(S[2 * sv + 2 * sw]), x2, y2);
-    }
+    double y[3];
+    if (layer == 0) stencil_layer<0>(L, sten, in, r0, xs[0], y);
+    else if (layer == 1) stencil_layer<1>(L, sten, in, r0, xs[1], y);
+    else stencil_layer<2>(L, sten, in, r0, xs[2], y);
+    __syncthreads();
+    double* sum = &xs[0][0][0];   // [3 layers][DOF of the work-group]
+#pragma unroll
+    for (int v = 0; v < 3; v++) sum[layer * 3 * kStenNodes + 3 * lane + v] = y[v];
+    __syncthreads();
+    const int64_t t = int64_t(r0) * 3 + threadIdx.x;
+    if (t >= L.n_nodes * 3) return;
     const double ith = L.cheb[0];
     const double c1 = step > 0 ? L.cheb[2 * step] : 0.0, c2 = step > 0 ? L.cheb[2 * step + 1] : 0.0;
-    mg_epilogue(L, mode, r * 3 + 0, y0, din, dout, c1, c2, ith);
-    mg_epilogue(L, mode, r * 3 + 1, y1, din, dout, c1, c2, ith);
-    mg_epilogue(L, mode, r * 3 + 2, y2, din, dout, c1, c2, ith);
+    const double s = (sum[threadIdx.x] + sum[3 * kStenNodes + threadIdx.x]) + sum[6 * kStenNodes + threadIdx.x];
+    mg_epilogue(L, mode, t, s, din, dout, c1, c2, ith);
 }
 
 // ---- the heat problem level as a stencil in lattice order ------------------
@@ -1534,7 +1608,7 @@ void launch_mg_gather_stencil3(const MGLevelArgs& L, const int32_t* rank_of_lat,
 }
 void launch_mg_stencil(const MGLevelArgs& L, const float* sten, int mode, int step, const double* din, double* dout,
                        const int* done, hipStream_t s) {
-    hipLaunchKernelGGL(k_mg_stencil, dim3(mg_blocks(L.n_nodes, 256)), dim3(256), 0, s, L, sten, mode, step, din,
+    hipLaunchKernelGGL(k_mg_stencil, dim3(mg_blocks(L.n_nodes, kStenNodes)), dim3(3 * kStenNodes), 0, s, L, sten, mode, step, din,
                        dout, done);
 }
 void launch_mg_to_stencil27(const MGLevelArgs& L, float* sten, hipStream_t s) {

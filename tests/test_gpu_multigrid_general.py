@@ -53,3 +53,23 @@ def test_distorted_hex8_multigrid(oracle, mastg, mesh):
     # (426 and 764 iterations at the two sizes)
     assert rm["iters"] <= 40 and rm["iters"] * 10 < rp["iters"], (rm["iters"], rp["iters"])
     ctx.close()
+
+
+# the stencil smoother takes 64 nodes a work-group and reads neighbours as runs
+# of 66: one node short of a work-group (63, the smallest lattice), a few with a
+# remainder (275, 637) and rows longer and shorter than a run (3045 nodes)
+@pytest.mark.parametrize("mesh", [(6, 2, 2), (10, 4, 4), (12, 6, 6), (28, 14, 6)])
+def test_stencil_smoother_edges(oracle, mastg, mesh):
+    print(f"[stencil smoother] distorted hex8 {mesh}", flush=True)
+    P0, P, a = distorted(oracle, *mesh, amp=0.25, seed=6)
+    desc = mastg.desc_from_arrays(mastg.HEX8_ELASTIC, a["xyz"], a["conn"], a["n_vars"], node_dof_base=a["node_base"],
+                                  constrained_dofs=np.nonzero(a["constrained"])[0], sides=P0.bsides(),
+                                  point_loads=a["point_load"], E=72e9, nu=0.33, penalty=3.0)
+    ctx = mastg.Context(desc)
+    ctx._keep = desc
+    ref = P.solve_elastic(1e-12)
+    r = ctx.design_eval(a["params"], solver=mastg.SOLVER_MG)
+    assert r["rel_res"] <= 1.5e-10 and r["iters"] <= 40, r["iters"]
+    assert abs(r["objective"] - ref["compliance"]) <= 1e-9 * ref["compliance"]
+    assert rel_err_floor(r["grad"], ref["dc"], floor=1e-6) <= 1e-7
+    ctx.close()
