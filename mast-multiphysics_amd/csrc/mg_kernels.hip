@@ -1109,20 +1109,42 @@ __device__ __forceinline__ int64_t mg_fine_index(const MGLevelArgs& F, int64_t p
     return (FL == FL_RANK ? int64_t(F.rank_of_lat[p]) : p) * NAV + v;
 }
 
+// The transfers take a thread per DOF: with a thread per node the chip is nearly
+// empty on the coarse levels and a thread's loads wait for each other (3
+// variables, 33x17x17 coarse nodes in 65x33x33: restriction 7.7 us against now
+// 4.8, prolongation 7.3 against 4.9; 65x33x33 in 129x65x65 14.1 / 12.9 and 15.9 /
+// 13.3; the plate's 33^2 in 65^2 7.7 / 5.1 and 6.4 / 3.7).
+// point and variable of thread t: planar levels by variable (coalesced per
+// component), the others as their vectors lie
+template <int NAV, int FL>
+__device__ __forceinline__ void mg_dof(uint32_t t, uint32_t n_nodes, uint32_t& p, int& v) {
+    if (FL == FL_PLANAR) {
+        v = int(t / n_nodes);
+        p = t - uint32_t(v) * n_nodes;
+    } else {
+        p = t / NAV;
+        v = int(t - p * NAV);
+    }
+}
+
 template <int DIM, int NAV, int FL>
 __global__ __launch_bounds__(256) void k_mg_restrict(MGLevelArgs F, MGLevelArgs Cl, const int* __restrict__ done) {
     if (done && *done) return;
-    const int64_t p = int64_t(blockIdx.x) * 256 + threadIdx.x;
-    if (p >= Cl.n_nodes) return;
+    const uint32_t t = blockIdx.x * 256 + threadIdx.x, nc = uint32_t(Cl.n_nodes);
+    if (t >= nc * NAV) return;
+    uint32_t p;
+    int v;
+    mg_dof<NAV, FL>(t, nc, p, v);
     // 32-bit index arithmetic (lattice point counts are below 2^31)
-    const uint32_t cx = uint32_t(Cl.nx + 1), cy = uint32_t(Cl.ny + 1), pu = uint32_t(p), pq = pu / cx;
-    const int I = int(pu - pq * cx), J = int(pq % cy), K = int(pq / cy);
+    const uint32_t cx = uint32_t(Cl.nx + 1), cy = uint32_t(Cl.ny + 1), pq = p / cx;
+    const int I = int(p - pq * cx), J = int(pq % cy), K = int(pq / cy);
     const uint32_t fx = uint32_t(F.nx + 1), fy = uint32_t(F.ny + 1);
     constexpr int NO = DIM == 3 ? 27 : 9;
+    const int64_t rc = int64_t(p) * NAV + v;
+    const bool con = Cl.con[rc];
+    const double dinv = Cl.dinv[rc], ith = Cl.cheb[0];
     // all loads are independent (unrolled, predicated) so they are in flight together
-    double sv[NAV];
-#pragma unroll
-    for (int v = 0; v < NAV; v++) sv[v] = 0.0;
+    double s = 0.0;
 #pragma unroll
     for (int o = 0; o < NO; o++) {
         const int oi = (o % 3) - 1, oj = ((o / 3) % 3) - 1, ok = DIM == 3 ? (o / 9) - 1 : 0;
@@ -1131,25 +1153,17 @@ __global__ __launch_bounds__(256) void k_mg_restrict(MGLevelArgs F, MGLevelArgs 
         // out-of-lattice points are clamped (valid address) and weighted 0
         const double w = in_lat ? (ok ? 0.5 : 1.0) * (oj ? 0.5 : 1.0) * (oi ? 0.5 : 1.0) : 0.0;
         const uint32_t fp = uint32_t(in_lat ? fi : 0) + fx * (uint32_t(in_lat ? fj : 0) + fy * uint32_t(in_lat ? fk : 0));
-#pragma unroll
-        for (int v = 0; v < NAV; v++) {
-            const int64_t rf = mg_fine_index<FL, NAV>(F, fp, v);
-            const double res = FL == FL_PLANAR ? double(F.res32[rf]) : F.res[rf];
-            sv[v] += (w * (1.0 - double(F.con[rf]))) * res;
-        }
+        const int64_t rf = mg_fine_index<FL, NAV>(F, fp, v);
+        const double res = FL == FL_PLANAR ? double(F.res32[rf]) : F.res[rf];
+        s += (w * (1.0 - double(F.con[rf]))) * res;
     }
     // and the coarse level's pre-smoothing start (x = 0, res = r, first
     // Chebyshev direction D^-1 r / theta)
-    const int64_t rc = p * NAV;
-    const double ith = Cl.cheb[0];
-#pragma unroll
-    for (int v = 0; v < NAV; v++) {
-        const double r = Cl.con[rc + v] ? 0.0 : sv[v];
-        Cl.r[rc + v] = r;
-        Cl.x[rc + v] = 0.0;
-        Cl.res[rc + v] = r;
-        Cl.da[rc + v] = Cl.dinv[rc + v] * r * ith;
-    }
+    const double r = con ? 0.0 : s;
+    Cl.r[rc] = r;
+    Cl.x[rc] = 0.0;
+    Cl.res[rc] = r;
+    Cl.da[rc] = dinv * r * ith;
 }
 
 // x_f += P (x_C + dlast_C) at unconstrained fine DOFs (tri/bilinear interpolation)
@@ -1157,16 +1171,20 @@ template <int DIM, int NAV, int FL>
 __global__ __launch_bounds__(256) void k_mg_prolong(MGLevelArgs F, MGLevelArgs Cl, const double* __restrict__ dlast,
                                                     const int* __restrict__ done) {
     if (done && *done) return;
-    const int64_t p = int64_t(blockIdx.x) * 256 + threadIdx.x;
-    if (p >= F.n_nodes) return;
+    const uint32_t t = blockIdx.x * 256 + threadIdx.x, nf = uint32_t(F.n_nodes);
+    if (t >= nf * NAV) return;
+    uint32_t p;
+    int v;
+    mg_dof<NAV, FL>(t, nf, p, v);
     // 32-bit index arithmetic (lattice point counts are below 2^31)
-    const uint32_t fx = uint32_t(F.nx + 1), fy = uint32_t(F.ny + 1), pu = uint32_t(p), pq = pu / fx;
-    const int fi = int(pu - pq * fx), fj = int(pq % fy), fk = int(pq / fy);
+    const uint32_t fx = uint32_t(F.nx + 1), fy = uint32_t(F.ny + 1), pq = p / fx;
+    const int fi = int(p - pq * fx), fj = int(pq % fy), fk = int(pq / fy);
     const uint32_t cx = uint32_t(Cl.nx + 1), cy = uint32_t(Cl.ny + 1);
+    const int64_t rf = mg_fine_index<FL, NAV>(F, p, v);
+    const bool con = F.con[rf];
+    const double x0 = FL == FL_PLANAR ? double(F.x32[rf]) : F.x[rf];
     constexpr int NQ = 1 << DIM;
-    double sv[NAV];
-#pragma unroll
-    for (int v = 0; v < NAV; v++) sv[v] = 0.0;
+    double s = 0.0;
 #pragma unroll
     for (int q = 0; q < NQ; q++) {
         const int a = q & 1, b = (q >> 1) & 1, c = DIM == 3 ? (q >> 2) : 0;
@@ -1176,20 +1194,12 @@ __global__ __launch_bounds__(256) void k_mg_prolong(MGLevelArgs F, MGLevelArgs C
         const double w = use ? ((fi & 1) ? 0.5 : 1.0) * ((fj & 1) ? 0.5 : 1.0) * ((fk & 1) ? 0.5 : 1.0) : 0.0;
         const uint32_t CI = uint32_t(min((fi >> 1) + a, Cl.nx)), CJ = uint32_t(min((fj >> 1) + b, Cl.ny)),
                        CK = uint32_t(min((fk >> 1) + c, Cl.nz));
-        const int64_t rc = int64_t(CI + cx * (CJ + cy * CK)) * NAV;
-        if (use)
-#pragma unroll
-            for (int v = 0; v < NAV; v++) sv[v] += w * (dlast ? Cl.x[rc + v] + dlast[rc + v] : Cl.x[rc + v]);
+        const int64_t rc = int64_t(CI + cx * (CJ + cy * CK)) * NAV + v;
+        if (use) s += w * (dlast ? Cl.x[rc] + dlast[rc] : Cl.x[rc]);
     }
-#pragma unroll
-    for (int v = 0; v < NAV; v++) {
-        const int64_t rf = mg_fine_index<FL, NAV>(F, p, v);
-        if (FL == FL_PLANAR) {
-            if (!F.con[rf]) F.x32[rf] += float(sv[v]);
-        } else {
-            if (!F.con[rf]) F.x[rf] += sv[v];
-        }
-    }
+    if (con) return;
+    if (FL == FL_PLANAR) F.x32[rf] = float(x0) + float(s);
+    else F.x[rf] = x0 + s;
 }
 
 // ---- coarsest level: dense inverse -------------------------------------------
@@ -1671,7 +1681,7 @@ void launch_mg_bsr(const MGLevelArgs& L, int mode, int step, const double* din, 
     }
 }
 void launch_mg_restrict(const MGLevelArgs& F, const MGLevelArgs& C, const int* done, hipStream_t s) {
-    const dim3 g(mg_blocks(C.n_nodes, 256));
+    const dim3 g(mg_blocks(C.n_nodes * C.nav, 256));
     const int fl = F.planar ? FL_PLANAR : F.rank_of_lat ? FL_RANK : FL_LAT;
     if (F.dim == 2) {
         if (fl == FL_RANK) hipLaunchKernelGGL((k_mg_restrict<2, 5, FL_RANK>), g, dim3(256), 0, s, F, C, done);
@@ -1687,7 +1697,7 @@ void launch_mg_restrict(const MGLevelArgs& F, const MGLevelArgs& C, const int* d
 }
 void launch_mg_prolong(const MGLevelArgs& F, const MGLevelArgs& C, const double* dlast, const int* done,
                        hipStream_t s) {
-    const dim3 g(mg_blocks(F.n_nodes, 256));
+    const dim3 g(mg_blocks(F.n_nodes * F.nav, 256));
     const int fl = F.planar ? FL_PLANAR : F.rank_of_lat ? FL_RANK : FL_LAT;
     if (F.dim == 2) {
         if (fl == FL_RANK) hipLaunchKernelGGL((k_mg_prolong<2, 5, FL_RANK>), g, dim3(256), 0, s, F, C, dlast, done);
