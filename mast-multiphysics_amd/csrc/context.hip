@@ -473,7 +473,10 @@ bool row_assembly_ok(mastg_ctx* c, bool fp32) {
 
 // ---- assembly: element kernel -> segmented scatter -> Jacobi diagonal, or
 // the fused row-owner kernel (hex8 elasticity)
-int assemble_active(mastg_ctx* c, const double* X_active, bool want_R, bool want_K, bool fp32 = false) {
+// (J_out: device memory for a copy of the values, *J_written whether the
+// assembly has written it)
+int assemble_active(mastg_ctx* c, const double* X_active, bool want_R, bool want_K, bool fp32 = false,
+                    double* J_out = nullptr, bool* J_written = nullptr) {
     if (!c->params_set) return fail(c, MASTG_ERR_INVALID, "design parameters not set");
     const Structure& S = c->S;
     if (want_K && row_assembly_ok(c, fp32)) {
@@ -501,6 +504,7 @@ int assemble_active(mastg_ctx* c, const double* X_active, bool want_R, bool want
         a.X = X_active;
         a.F = c->F.as<double>();
         a.val = c->val.as<double>();
+        a.val2 = J_out;
         a.R = want_R ? c->vtmp.as<double>() : nullptr;
         a.dinv = c->dinv.as<double>();
         // the class kernel's row plan: at most 8 elements per node
@@ -521,6 +525,7 @@ int assemble_active(mastg_ctx* c, const double* X_active, bool want_R, bool want
             TimedRegion t(c, 0);
             launch_hex8_row_assemble(a, int(S.max_blocks_per_row), c->stream);
         }
+        if (J_written) *J_written = J_out != nullptr;
         c->assembled = true;
         c->val32_valid = false;
         c->kel64_valid = false;
@@ -2139,6 +2144,17 @@ int mastg_set_params(mastg_ctx* c, const double* p, int where) {
     return MASTG_OK;
 }
 
+// p can be written by this context's kernels: memory of its own device (a copy
+// reaches more: other devices without peer access, any alignment)
+static bool kernel_writable(const mastg_ctx* c, const void* p) {
+    hipPointerAttribute_t at{}, own{};
+    if (hipPointerGetAttributes(&at, p) != hipSuccess || hipPointerGetAttributes(&own, c->xyz.p) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return at.type == hipMemoryTypeDevice && at.device == own.device && reinterpret_cast<uintptr_t>(p) % sizeof(double) == 0;
+}
+
 int mastg_assemble(mastg_ctx* c, const double* X, double* R, double* J, int where, int prec) {
     if (!c) return MASTG_ERR_INVALID;
     if (prec != MASTG_ELEM_FP64 && prec != MASTG_ELEM_FP32)
@@ -2148,9 +2164,11 @@ int mastg_assemble(mastg_ctx* c, const double* X, double* R, double* J, int wher
     const Structure& S = c->S;
     double* Xa = c->vb.as<double>();
     TRY(to_active(c, X, where, Xa));
-    TRY(assemble_active(c, X ? Xa : nullptr, R != nullptr, true, prec == MASTG_ELEM_FP32));
+    double* J_out = where != MASTG_HOST && J && kernel_writable(c, J) ? J : nullptr;
+    bool J_written = false;
+    TRY(assemble_active(c, X ? Xa : nullptr, R != nullptr, true, prec == MASTG_ELEM_FP32, J_out, &J_written));
     if (R) TRY(from_active(c, c->vtmp.as<double>(), R, where));
-    if (J) {
+    if (J && !J_written) {
         HIPC(c, hipMemcpyAsync(J, c->val.p, S.nnz * sizeof(double),
                                where == MASTG_HOST ? hipMemcpyDeviceToHost : hipMemcpyDeviceToDevice,
                                c->stream));

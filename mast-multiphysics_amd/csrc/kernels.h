@@ -81,6 +81,7 @@ struct Hex8RowArgs {
     const double* X;          // [n_active] state or null (no residual from the elements)
     const double* F;          // [n_active] loads or null
     double* val;              // CSR values
+    double* val2;             // a second copy of them (the caller's) or null
     double* R;                // [n_active] residual or null
     double* dinv;             // [n_active] inverse diagonal or null
     // row plan of the class kernel (null: positions searched per pass):
