@@ -1122,10 +1122,11 @@ __global__ __launch_bounds__(256) void k_spmv_csr_dot(CGArgs C, const double* __
 
 // The iteration's scalars have no kernels of their own: each work-group sums
 // the partials of the kernel before it (a few KB from L2, about 1 us) instead
-// of waiting for a launch that does (2.2-3.6 us and a graph node's gap; the
-// iteration on 23,805 hex8 cells with the element-wise product 25.9 -> 23.4 us).  A scalar that a kernel
-// updates is never one that its work-groups read: `iter` moves in k_cg_p,
-// `next` in k_cg_update, and r.z of iteration i lives in rz2[i & 1].
+// of waiting for a launch that does (2.2-3.6 us and a graph node's gap; an
+// iteration on 23,805 hex8 cells with the element-wise product 25.9 -> 23.4
+// us).  A scalar that a kernel updates is never one that its work-groups read:
+// `iter` moves in k_cg_p, `next` in k_cg_update, and r.z of iteration i lives
+// in rz2[i & 1].
 
 // alpha = r.z / p.q; x += alpha p; r -= alpha q; z = dinv r; partials of r.r, r.z
 __global__ __launch_bounds__(256) void k_cg_update(CGArgs C) {
