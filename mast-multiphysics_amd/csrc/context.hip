@@ -139,6 +139,7 @@ struct mastg_ctx {
     // matrix-free operator data (hex8 congruence classes)
     DevBuf Khat, sE, eclass, nodecon, Fel;
     MFLattice mf_lat;
+    int device = -1;            // the buffers' device, once asked for
     DevBuf heat_geo;            // heat: per congruence class gradients and JxW
     DevBuf Khat32;              // FP32 copy of Khat (lattice smoothing)
     bool is_box = false;        // Khat is an axis-aligned box's: box, box32
@@ -2146,13 +2147,17 @@ int mastg_set_params(mastg_ctx* c, const double* p, int where) {
 
 // p can be written by this context's kernels: memory of its own device (a copy
 // reaches more: other devices without peer access, any alignment)
-static bool kernel_writable(const mastg_ctx* c, const void* p) {
-    hipPointerAttribute_t at{}, own{};
-    if (hipPointerGetAttributes(&at, p) != hipSuccess || hipPointerGetAttributes(&own, c->xyz.p) != hipSuccess) {
+static bool kernel_writable(mastg_ctx* c, const void* p) {
+    hipPointerAttribute_t at{};
+    if (c->device < 0) {   // where the context's buffers are
+        if (hipPointerGetAttributes(&at, c->xyz.p) == hipSuccess) c->device = at.device;
+        else (void)hipGetLastError();
+    }
+    if (hipPointerGetAttributes(&at, p) != hipSuccess) {
         (void)hipGetLastError();
         return false;
     }
-    return at.type == hipMemoryTypeDevice && at.device == own.device && reinterpret_cast<uintptr_t>(p) % sizeof(double) == 0;
+    return at.type == hipMemoryTypeDevice && at.device == c->device && reinterpret_cast<uintptr_t>(p) % sizeof(double) == 0;
 }
 
 int mastg_assemble(mastg_ctx* c, const double* X, double* R, double* J, int where, int prec) {
@@ -2164,7 +2169,8 @@ int mastg_assemble(mastg_ctx* c, const double* X, double* R, double* J, int wher
     const Structure& S = c->S;
     double* Xa = c->vb.as<double>();
     TRY(to_active(c, X, where, Xa));
-    double* J_out = where != MASTG_HOST && J && kernel_writable(c, J) ? J : nullptr;
+    const bool rows = row_assembly_ok(c, prec == MASTG_ELEM_FP32);
+    double* J_out = where != MASTG_HOST && J && rows && kernel_writable(c, J) ? J : nullptr;
     bool J_written = false;
     TRY(assemble_active(c, X ? Xa : nullptr, R != nullptr, true, prec == MASTG_ELEM_FP32, J_out, &J_written));
     if (R) TRY(from_active(c, c->vtmp.as<double>(), R, where));

@@ -524,8 +524,7 @@ void launch_pcg_recheck(const CGArgs& c, hipStream_t s);
 // out = x0 + dlast (a V-cycle's level-0 output), skipped when *done
 void launch_mg_combine(int64_t n, const double* x0, const double* dlast, double* out, const int* done,
                        hipStream_t s);
-// pieces of the CG iteration shared with the preconditioned variant
-void launch_mf_elem(const CGArgs& c, const double* x, hipStream_t s);   // element phase only
-void launch_cg_op(const CGArgs& c, hipStream_t s);                      // q = A p, partials of p.q
+// the CG iteration's product, shared with the preconditioned variant
+void launch_cg_op(const CGArgs& c, hipStream_t s);   // q = A p, partials of p.q
 
 }  // namespace mastg

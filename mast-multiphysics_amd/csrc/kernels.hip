@@ -1650,13 +1650,6 @@ void launch_mf_apply(const CGArgs& c, const double* x_elem, const double* x_node
 void launch_mask_constrained(int64_t n, const uint8_t* con, double* x, hipStream_t s) {
     hipLaunchKernelGGL(k_mask_constrained, dim3(blocks_for(n, 256)), dim3(256), 0, s, n, con, x);
 }
-void launch_mf_elem(const CGArgs& c, const double* x, hipStream_t s) {
-    const unsigned ge = blocks_for(c.mf.n_elems, 256);
-    if (c.mf.n_classes == 1)
-        hipLaunchKernelGGL(k_hex8_mf_elem<true>, dim3(ge), dim3(256), 0, s, c, x);
-    else
-        hipLaunchKernelGGL(k_hex8_mf_elem<false>, dim3(ge), dim3(256), 0, s, c, x);
-}
 void launch_cg_op(const CGArgs& c, hipStream_t s) {
     if (c.use_mf == 1)
         mf_dispatch(c, c.p, c.p, c.q, 1, s);
