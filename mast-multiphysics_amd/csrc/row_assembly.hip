@@ -495,7 +495,8 @@ __device__ __forceinline__ void ready(int v) { asm volatile("" ::"v"(v)); }
 
 constexpr int kPlanRun = 32;   // nodes per work-group at most (a lane holds each one's pointers)
 
-template <int NP, bool ONE>
+// TWO: both copies of the values, as whole lines through LDS
+template <int NP, bool ONE, bool TWO>
 __global__ __launch_bounds__(64) void k_hex8_row_assemble_plan(Hex8RowArgs A) {
     constexpr int MAXB = NP * 64 / 3;
     constexpr int kZero = 64;   // kh row of zeros: the slots that do not touch a neighbour
@@ -504,7 +505,7 @@ __global__ __launch_bounds__(64) void k_hex8_row_assemble_plan(Hex8RowArgs A) {
     // the run's residual and inverse diagonal, written out once at its end
     // (node by node, 24-byte pieces of lines that leave L2 in between)
     __shared__ double sres[kPlanRun * 3], sdinv[kPlanRun * 3];
-    __shared__ double stage[MAXB * 9];   // the node's values, in the order they are written
+    __shared__ double stage[TWO ? MAXB * 9 : 1];   // TWO: the node's values, in the order they are written
     const int lane = threadIdx.x;
     for (int t = lane; t < 65 * 9; t += 64) kh[t] = (ONE && t < 576) ? A.Khat[t] : 0.0;
     for (int t = lane; t < MAXB * 8; t += 64) cont[t] = kZero;
@@ -666,24 +667,30 @@ __global__ __launch_bounds__(64) void k_hex8_row_assemble_plan(Hex8RowArgs A) {
             const int k = pk[jp], v = pv[jp];
             if (p < npair) {
 #pragma unroll
-                for (int w = 0; w < 3; w++) stage[3 * p + w] = vals[jp][w];
+                for (int w = 0; w < 3; w++) {
+                    if (TWO) stage[3 * p + w] = vals[jp][w];
+                    else A.val[start + 3 * p + w] = vals[jp][w];
+                }
                 if (k == kd) {
                     const double d = v == 0 ? vals[jp][0] : v == 1 ? vals[jp][1] : vals[jp][2];
                     sdinv[j * 3 + v] = 1.0 / d;
                 }
             }
         }
-        __syncthreads();
-        // whole lines: 64 consecutive values per store (a lane's own three
-        // values are 24 bytes apart from the next lane's: three stores that each
-        // touch every line; with both copies of the values 346 us, now 327)
+        if constexpr (TWO) {
+            __syncthreads();
+            // 64 consecutive values per store: a lane's own three are 24 bytes
+            // from the next lane's, three stores that each touch every line.
+            // 97x47x45 cells: 346 us, staged 327.  With one copy the LDS costs
+            // more waves than the lines save: 128x64x64 cells 563 us, staged 601.
 #pragma unroll
-        for (int i = 0; i < (MAXB * 9 + 63) / 64; i++) {
-            const int q = lane + 64 * i;
-            if (q < 3 * npair) {
-                const double v = stage[q];
-                A.val[start + q] = v;
-                if (A.val2) A.val2[start + q] = v;
+            for (int i = 0; i < (MAXB * 9 + 63) / 64; i++) {
+                const int q = lane + 64 * i;
+                if (q < 3 * npair) {
+                    const double v = stage[q];
+                    A.val[start + q] = v;
+                    A.val2[start + q] = v;
+                }
             }
         }
         if (kd < 0 && lane < 3) sdinv[j * 3 + lane] = 0.0;
@@ -701,6 +708,12 @@ __global__ __launch_bounds__(64) void k_hex8_row_assemble_plan(Hex8RowArgs A) {
     }
 }
 
+template <int NP, bool ONE>
+void launch_plan(const Hex8RowArgs& a, dim3 g, hipStream_t s) {
+    if (a.val2) hipLaunchKernelGGL((k_hex8_row_assemble_plan<NP, ONE, true>), g, dim3(64), 0, s, a);
+    else hipLaunchKernelGGL((k_hex8_row_assemble_plan<NP, ONE, false>), g, dim3(64), 0, s, a);
+}
+
 }  // namespace
 
 int hex8_row_assembly_max_blocks() { return kRowMaxBlocks; }
@@ -715,11 +728,11 @@ void launch_hex8_row_assemble(const Hex8RowArgs& a, int max_blocks_per_row, hipS
                                                  (a.n_nodes + kPlanRun - 1) / kPlanRun)));
         const bool two = max_blocks_per_row <= 42;
         if (a.n_classes == 1) {
-            if (two) hipLaunchKernelGGL((k_hex8_row_assemble_plan<2, true>), gp, dim3(64), 0, s, a);
-            else hipLaunchKernelGGL((k_hex8_row_assemble_plan<3, true>), gp, dim3(64), 0, s, a);
+            if (two) launch_plan<2, true>(a, gp, s);
+            else launch_plan<3, true>(a, gp, s);
         } else {
-            if (two) hipLaunchKernelGGL((k_hex8_row_assemble_plan<2, false>), gp, dim3(64), 0, s, a);
-            else hipLaunchKernelGGL((k_hex8_row_assemble_plan<3, false>), gp, dim3(64), 0, s, a);
+            if (two) launch_plan<2, false>(a, gp, s);
+            else launch_plan<3, false>(a, gp, s);
         }
         return;
     }
