@@ -1234,7 +1234,8 @@ bool lattice_args(mastg_ctx* c, CGArgs& a) {
 // matrix-free hex8 problem level (FP32) returns the output itself, with the
 // partial sums of r . output in a.part0.  started: within a CG iteration, whose
 // convergence test then runs beside the first kernel (and whose update has
-// written the FP32 level's pre-smoothing start)
+// written the FP32 level's pre-smoothing start); done is then the test's done_z,
+// which the first kernel does not look at
 const void* mg_vcycle(mastg_ctx* c, const CGArgs& a, const int* done, hipStream_t s, const double* r0 = nullptr,
                       bool started = false) {
     const int nl = int(c->mg.size());
@@ -1350,7 +1351,7 @@ void mg_rz(mastg_ctx* c, const CGArgs& a, const void* dl, hipStream_t s) {
 // an iteration has no kernel for scalars alone: each kernel sums the partials of
 // the one before it
 void mg_pcg_iteration(mastg_ctx* c, const CGArgs& a, hipStream_t s) {
-    const int* done = &a.S->done;
+    const int* done = &a.S->done_z;
     const MGLevelArgs& L0 = c->mg[0]->a;
     if (L0.planar) {   // the lattice solver
         launch_lattice_apply(a, a.p, a.q, s);
@@ -1367,7 +1368,7 @@ void mg_pcg_iteration(mastg_ctx* c, const CGArgs& a, hipStream_t s) {
 
 // z = M r and p = z, from the residual in a.r (the start of PCG, and its restarts)
 void mg_pcg_begin(mastg_ctx* c, const CGArgs& a, hipStream_t s) {
-    const void* z = mg_vcycle(c, a, &a.S->done, s);
+    const void* z = mg_vcycle(c, a, &a.S->done_z, s);
     if (c->mg[0]->a.planar) {
         launch_pcg_p(a, static_cast<const float*>(z), int(lattice_partials(a.lat)), 1, s);
         return;
@@ -1536,19 +1537,19 @@ int ensure_bicg(mastg_ctx* c) {
 // BiCGStab iteration right-preconditioned by the multigrid V-cycle: ph = M p,
 // sh = M s replace the Jacobi scalings of the plain iteration
 void mg_bicg_iteration(mastg_ctx* c, const BiCGArgs& a, hipStream_t s) {
-    const int* done = &a.S->done;
     const CGArgs none{};
     const int64_t n = c->S.n_active;
     launch_bicg_part(a, 0, s);
     // (plate and heat: FP64 problem-level state)
     const MGLevelDev& D0 = *c->mg[0];
-    auto combine = [&](const double* dl, double* out) {
+    auto precondition = [&](const double* in, double* out, const int* done) {
+        const double* dl = static_cast<const double*>(mg_vcycle(c, none, done, s, in));
         if (D0.lat0) launch_mg_combine_rank(D0.a.n_nodes, D0.a.nav, D0.a.rank_of_lat, D0.a.x, dl, out, done, s);
         else launch_mg_combine(n, D0.a.x, dl, out, done, s);
     };
-    combine(static_cast<const double*>(mg_vcycle(c, none, done, s, a.p)), a.ph);
+    precondition(a.p, a.ph, &a.S->done_p);
     launch_bicg_part(a, 1, s);
-    combine(static_cast<const double*>(mg_vcycle(c, none, done, s, a.s)), a.sh);
+    precondition(a.s, a.sh, &a.S->done);
     launch_bicg_part(a, 2, s);
 }
 

@@ -91,17 +91,27 @@ __device__ __forceinline__ void block_max_store(double v, double* partials, int 
 }
 
 // one work-group of 256: ||r||^2 of the updated residual, the iteration count
-// and convergence
+// and convergence (after an outcome: handed on)
 __device__ __forceinline__ void pcg_check_block(const CGCheck& C) {
+    CGScalars* S = C.S;
+    const int was = S->done_r;
+    if (was) {
+        if (threadIdx.x == 0) S->done_z = was;
+        return;
+    }
     const double rr = reduce_partials(C.part, C.n);
     if (threadIdx.x == 0) {
-        CGScalars* S = C.S;
+        const int it = S->iter + 1;
         S->rr = rr;
-        S->iter += 1;
-        if (!isfinite(rr)) S->done = 4;
-        else if (rr <= S->tol2 * S->bb) S->done = 1;
-        else if (S->iter >= S->max_it) S->done = 2;
+        S->iter = it;
+        S->done_z = !isfinite(rr) ? 4 : rr <= S->tol2 * S->bb ? 1 : it >= S->max_it ? 2 : 0;
     }
+}
+
+// whether a V-cycle kernel that may carry the convergence test has nothing to do
+// (the test's own flag is written beside it)
+__device__ __forceinline__ bool vcycle_done(const CGCheck& C, const int* done) {
+    return C.S ? C.S->done_r != 0 : done && *done;
 }
 
 // the coefficients of a lattice smoothing pass, and its update of one value

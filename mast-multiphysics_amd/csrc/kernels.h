@@ -128,15 +128,23 @@ struct ScatterArgs {
     double* val;
 };
 
+// The outcome (0: go on) moves along with the iteration's launches, so that no
+// launch tests a flag that it writes: a work-group's waves read it one by one,
+// and one that saw it set by another work-group would leave the rest at their
+// reductions.  `done` is written by the last kernel (p) and tested by the product
+// and the update of x and r; the update writes done_r (`done`, or a breakdown of
+// its own), which plain CG's p kernel tests, or PCG's convergence test; that one
+// writes done_z, which the rest of the V-cycle and PCG's p kernel test.
 struct CGScalars {
     double rr, bb, tol2;
     int iter, max_it, done;
     int next;        // the iteration that the vector kernels of plain CG are in
     double rz2[2];   // r.z of iteration i in rz2[i & 1]
+    int done_r, done_z;
 };
 
 // the convergence test of a CG iteration, done by one work-group beside other
-// work: ||r||^2 from its partial sums (S null: no test)
+// work: ||r||^2 from its partial sums (S null: no test); the outcome into done_z
 struct CGCheck {
     CGScalars* S;
     const double* part;
@@ -240,7 +248,10 @@ struct CGArgs {
 // right-preconditioned BiCGStab + Jacobi on a scalar CSR (PETSc KSPBCGS role)
 struct BiCGScalars {
     double rho, rho_old, alpha, omega, rr, bb, tol2;
-    int iter, max_it, done, pad;
+    // as in CGScalars: `done` is tested from the t product to the next p kernel,
+    // which writes done_p, tested from the v product to the s kernel, which
+    // writes `done`
+    int iter, max_it, done, done_p;
 };
 struct BiCGArgs {
     int64_t n;
@@ -399,7 +410,8 @@ void launch_mg_dense_gather(const MGLevelArgs& L, double* A, hipStream_t s);
 int64_t mg_invert_work(int n);
 double* mg_invert_input(int n, double* A, double* W);
 void launch_mg_invert(int n, double* A, double* W, hipStream_t s);
-// V-cycle pieces; every kernel returns at once when *done != 0 (done may be null)
+// V-cycle pieces; every kernel returns at once when *done != 0 (done may be
+// null), one with a convergence test (check.S) when check.S->done_r != 0
 // the problem level's start; a level in lattice order takes its right side from
 // the rank-ordered src (null: L.r); with CG's convergence test when check.S
 // (not for planar levels)

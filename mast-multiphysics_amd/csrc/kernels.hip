@@ -1125,21 +1125,26 @@ __global__ __launch_bounds__(256) void k_spmv_csr_dot(CGArgs C, const double* __
 // of waiting for a launch that does (2.2-3.6 us and a graph node's gap; an
 // iteration on 23,805 hex8 cells with the element-wise product 25.9 -> 23.4
 // us).  A scalar that a kernel updates is never one that its work-groups read:
-// `iter` moves in k_cg_p, `next` in k_cg_update, and r.z of iteration i lives
-// in rz2[i & 1].
+// `iter` moves in k_cg_p, `next` in k_cg_update, r.z of iteration i lives in
+// rz2[i & 1], and the outcome goes to and fro: k_cg_update tests `done` and
+// writes done_r, k_cg_p the other way round.
 
 // alpha = r.z / p.q; x += alpha p; r -= alpha q; z = dinv r; partials of r.r, r.z
 __global__ __launch_bounds__(256) void k_cg_update(CGArgs C) {
     CGScalars* S = C.S;
-    if (S->done) return;
-    const double pq = reduce_partials(C.part0, C.nparts_op);
-    if (!(pq > 0.0) || !isfinite(pq)) {   // breakdown / NaN, the same in every work-group
-        if (blockIdx.x == 0 && threadIdx.x == 0) S->done = 3;
+    const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
+    const int was = S->done;
+    if (was) {
+        if (lead) S->done_r = was;
         return;
     }
+    const double pq = reduce_partials(C.part0, C.nparts_op);
+    const bool bad = !(pq > 0.0) || !isfinite(pq);   // breakdown / NaN, the same in every work-group
+    if (lead) S->done_r = bad ? 3 : 0;
+    if (bad) return;
     const int it = S->iter;
     const double a = S->rz2[it & 1] / pq;
-    if (blockIdx.x == 0 && threadIdx.x == 0) S->next = it + 1;
+    if (lead) S->next = it + 1;
     double rz = 0.0, rr = 0.0;
     for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < C.n; i += int64_t(gridDim.x) * 256) {
         C.x[i] += a * C.p[i];
@@ -1159,17 +1164,22 @@ __global__ __launch_bounds__(256) void k_cg_update(CGArgs C) {
 // last r.z; p = z + beta p
 __global__ __launch_bounds__(256) void k_cg_p(CGArgs C) {
     CGScalars* S = C.S;
-    if (S->done) return;
+    const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
+    const int was = S->done_r;
+    if (was) {
+        if (lead) S->done = was;
+        return;
+    }
     const double2 sums = reduce_partials2(C.part1, C.part1 + C.nvec, C.nvec);
     const double rr = sums.x, rz = sums.y;
     const int it = S->next;
     const int done = !isfinite(rr) ? 4 : rr <= S->tol2 * S->bb ? 1 : it >= S->max_it ? 2 : 0;
     const double b = rz / S->rz2[(it + 1) & 1];
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (lead) {
         S->rr = rr;
         S->rz2[it & 1] = rz;
         S->iter = it;
-        if (done) S->done = done;
+        S->done = done;
     }
     if (done) return;
     for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < C.n; i += int64_t(gridDim.x) * 256)
@@ -1298,12 +1308,13 @@ __global__ __launch_bounds__(256) void k_copy_f64(int64_t n2, const double2* __r
 
 // ------------------------------------------------- BiCGStab (FP64 CSR) ----
 // y = A x with SW lanes per row; optional partials sum(y.w1) -> part0 and
-// sum(y.y) -> part1 (per block).  Stops immediately once the solver is done.
+// sum(y.y) -> part1 (per block).  Stops immediately once the solver is done
+// (*over: the outcome as of this launch).
 template <int SW>
 __global__ __launch_bounds__(256) void k_spmv_csr_gen(BiCGArgs B, const double* __restrict__ x,
                                                       double* __restrict__ y, const double* __restrict__ w1,
-                                                      int want_yy) {
-    if (B.S->done) return;
+                                                      int want_yy, const int* __restrict__ over) {
+    if (*over) return;
     const int sub = threadIdx.x & (SW - 1);
     double d1 = 0.0, d2 = 0.0;
     const int64_t rows_per_grid = (int64_t(gridDim.x) * 256) / SW;
@@ -1329,7 +1340,8 @@ __global__ __launch_bounds__(256) void k_spmv_csr_gen(BiCGArgs B, const double* 
 
 // The scalars are folded into the vector kernels as in CG: each work-group sums
 // the partials itself, and a kernel writes no scalar that its work-groups read
-// (k_bicg_p: rho; k_bicg_s: alpha, rho_old; k_bicg_xr: omega, iter).  Partials:
+// (k_bicg_p: rho, done_p; k_bicg_s: alpha, rho_old, done; k_bicg_xr: omega, iter;
+// tested: done, done_p, done).  Partials:
 // r.r after the operator's in part0, r0.r after the operator's in part1.
 __global__ __launch_bounds__(256) void k_bicg_start(BiCGArgs B, const double* __restrict__ b) {
     double bb = 0.0;
@@ -1362,16 +1374,21 @@ __device__ __forceinline__ int bicg_outcome(const BiCGScalars* S, double rr) {
 // convergence; rho, beta; p = r + beta (p - omega v); ph = dinv p
 __global__ __launch_bounds__(256) void k_bicg_p(BiCGArgs B) {
     BiCGScalars* S = B.S;
-    if (S->done) return;
+    const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
+    const int was = S->done;
+    if (was) {
+        if (lead) S->done_p = was;
+        return;
+    }
     const double2 sums = reduce_partials2(B.part0 + B.nparts, B.part1 + B.nparts, B.nvec);
     const double rr = sums.x, rho = sums.y;
     const int done = bicg_outcome(S, rr);
     const double om = S->omega;
     const double beta = (rho / S->rho_old) * (S->alpha / om);
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (lead) {
         S->rr = rr;
         S->rho = rho;
-        if (done) S->done = done;
+        S->done_p = done;
     }
     if (done) return;
     for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < B.n; i += int64_t(gridDim.x) * 256) {
@@ -1384,14 +1401,19 @@ __global__ __launch_bounds__(256) void k_bicg_p(BiCGArgs B) {
 // alpha = rho / r0.v; s = r - alpha v ; sh = dinv s
 __global__ __launch_bounds__(256) void k_bicg_s(BiCGArgs B) {
     BiCGScalars* S = B.S;
-    if (S->done) return;
+    const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
+    const int was = S->done_p;
+    if (was) {
+        if (lead) S->done = was;
+        return;
+    }
     const double r0v = reduce_partials(B.part0, B.nparts);
     const bool bad = !(r0v != 0.0) || !isfinite(r0v);
     const double rho = S->rho, al = rho / r0v;
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (lead) {
         S->alpha = al;
         S->rho_old = rho;
-        if (bad) S->done = 3;
+        S->done = bad ? 3 : 0;
     }
     if (bad) return;
     for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < B.n; i += int64_t(gridDim.x) * 256) {
@@ -1590,13 +1612,13 @@ void launch_cg_start(const CGArgs& c, const double* b, double tol2, int max_it, 
     hipLaunchKernelGGL(k_cg_start_scalars, dim3(1), dim3(256), 0, s, c, tol2, max_it);
 }
 static void spmv_gen(const BiCGArgs& B, const double* x, double* y, const double* w1, int want_yy,
-                     hipStream_t s) {
+                     const int* over, hipStream_t s) {
     switch (B.spmv_sw) {
-        case 4: hipLaunchKernelGGL(k_spmv_csr_gen<4>, dim3(B.nparts), dim3(256), 0, s, B, x, y, w1, want_yy); break;
-        case 8: hipLaunchKernelGGL(k_spmv_csr_gen<8>, dim3(B.nparts), dim3(256), 0, s, B, x, y, w1, want_yy); break;
-        case 32: hipLaunchKernelGGL(k_spmv_csr_gen<32>, dim3(B.nparts), dim3(256), 0, s, B, x, y, w1, want_yy); break;
-        case 64: hipLaunchKernelGGL(k_spmv_csr_gen<64>, dim3(B.nparts), dim3(256), 0, s, B, x, y, w1, want_yy); break;
-        default: hipLaunchKernelGGL(k_spmv_csr_gen<16>, dim3(B.nparts), dim3(256), 0, s, B, x, y, w1, want_yy); break;
+        case 4: hipLaunchKernelGGL(k_spmv_csr_gen<4>, dim3(B.nparts), dim3(256), 0, s, B, x, y, w1, want_yy, over); break;
+        case 8: hipLaunchKernelGGL(k_spmv_csr_gen<8>, dim3(B.nparts), dim3(256), 0, s, B, x, y, w1, want_yy, over); break;
+        case 32: hipLaunchKernelGGL(k_spmv_csr_gen<32>, dim3(B.nparts), dim3(256), 0, s, B, x, y, w1, want_yy, over); break;
+        case 64: hipLaunchKernelGGL(k_spmv_csr_gen<64>, dim3(B.nparts), dim3(256), 0, s, B, x, y, w1, want_yy, over); break;
+        default: hipLaunchKernelGGL(k_spmv_csr_gen<16>, dim3(B.nparts), dim3(256), 0, s, B, x, y, w1, want_yy, over); break;
     }
 }
 void launch_bicg_start(const BiCGArgs& a, const double* b, double tol2, int max_it, hipStream_t s) {
@@ -1607,10 +1629,10 @@ void launch_bicg_part(const BiCGArgs& a, int part, hipStream_t s) {
     if (part == 0) {
         hipLaunchKernelGGL(k_bicg_p, dim3(a.nvec), dim3(256), 0, s, a);
     } else if (part == 1) {
-        spmv_gen(a, a.ph, a.v, a.r0, 0, s);
+        spmv_gen(a, a.ph, a.v, a.r0, 0, &a.S->done_p, s);
         hipLaunchKernelGGL(k_bicg_s, dim3(a.nvec), dim3(256), 0, s, a);
     } else {
-        spmv_gen(a, a.sh, a.t, a.s, 1, s);
+        spmv_gen(a, a.sh, a.t, a.s, 1, &a.S->done, s);
         hipLaunchKernelGGL(k_bicg_xr, dim3(a.nvec), dim3(256), 0, s, a);
     }
 }

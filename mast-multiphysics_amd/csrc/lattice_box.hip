@@ -243,7 +243,6 @@ __global__ __launch_bounds__(256) void k_box_apply(LatticeOpArgs O, const double
 // S.check, only decides on convergence
 template <int NL>
 __global__ __launch_bounds__(256) void k_box_smooth(LatticeOpArgs O, LatSmooth S, const int* __restrict__ done) {
-    if (done && *done) return;
     unsigned nb = gridDim.x;
     if (S.check.S) {
         nb--;
@@ -252,6 +251,7 @@ __global__ __launch_bounds__(256) void k_box_smooth(LatticeOpArgs O, LatSmooth S
             return;
         }
     }
+    if (vcycle_done(S.check, done)) return;
     const int64_t plane = int64_t(O.nx + 1) * (O.ny + 1), n_lat = plane * (O.nz + 1);
     const uint32_t w = uint32_t(xcd_block(blockIdx.x, nb)) * 4 + (threadIdx.x >> 6);
     const BoxPoint b = box_point(O, w, threadIdx.x & 63, NL);

@@ -212,12 +212,12 @@ __device__ __forceinline__ void mg_epilogue(const MGLevelArgs& L, int mode, int6
 __global__ __launch_bounds__(256) void k_mg_pre_init(MGLevelArgs L, const double* __restrict__ src,
                                                      const int32_t* __restrict__ rank_of_lat, CGCheck check,
                                                      const int* __restrict__ done) {
-    if (done && *done) return;
     const int64_t nb = gridDim.x - (check.S ? 1 : 0);
     if (int64_t(blockIdx.x) == nb) {
         pcg_check_block(check);
         return;
     }
+    if (vcycle_done(check, done)) return;
     const double ith = L.cheb[0];
     for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < L.n_nodes * L.nav; i += nb * 256) {
         double r;
@@ -238,12 +238,12 @@ __global__ __launch_bounds__(256) void k_mg_pre_init(MGLevelArgs L, const double
 // a thread per DOF (row v of node n's inverse block), so that a wave's loads
 // of the blocks and of r cover contiguous memory
 __global__ __launch_bounds__(256) void k_mg_pre_init_blk5(MGLevelArgs L, CGCheck check, const int* __restrict__ done) {
-    if (done && *done) return;
     const int64_t nb = gridDim.x - (check.S ? 1 : 0);
     if (int64_t(blockIdx.x) == nb) {
         pcg_check_block(check);
         return;
     }
+    if (vcycle_done(check, done)) return;
     const double ith = L.cheb[0];
     for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < L.n_nodes * 5; i += nb * 256) {
         const int64_t n = i / 5;
@@ -857,7 +857,6 @@ __global__ __launch_bounds__(256) void k_lattice_apply(CGArgs C, const double* _
 // the convergence test stay FP64.  The last work-group, if S.check, only decides
 // on convergence.
 __global__ __launch_bounds__(256) void k_lattice_smooth(LatticeOpArgs O, LatSmooth S, const int* __restrict__ done) {
-    if (done && *done) return;
     unsigned nb = gridDim.x;
     if (S.check.S) {
         nb--;
@@ -866,6 +865,7 @@ __global__ __launch_bounds__(256) void k_lattice_smooth(LatticeOpArgs O, LatSmoo
             return;
         }
     }
+    if (vcycle_done(S.check, done)) return;
     const int64_t n_lat = int64_t(O.nx + 1) * (O.ny + 1) * (O.nz + 1);
     const int64_t t = xcd_block(blockIdx.x, nb) * 256 + threadIdx.x, p = t < n_lat ? t : 0;
     int i, j, k, cnt;
@@ -1368,22 +1368,26 @@ __global__ __launch_bounds__(256) void k_mg_coarse_solve(int n, const double* __
 
 // ---- preconditioned CG ---------------------------------------------------------
 // alpha = r.z / p.q, p.q from the operator's partials, summed by every
-// work-group (a launch less than a kernel for alpha); false: breakdown / NaN,
-// the same in every work-group
+// work-group (a launch less than a kernel for alpha); false: over, or breakdown /
+// NaN, the same in every work-group
 __device__ __forceinline__ bool pcg_alpha(const CGArgs& C, double& a) {
     CGScalars* S = C.S;
-    const double pq = reduce_partials(C.part0, C.nparts_op);
-    if (!(pq > 0.0) || !isfinite(pq)) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) S->done = 3;
+    const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
+    const int was = S->done;
+    if (was) {
+        if (lead) S->done_r = was;
         return false;
     }
+    const double pq = reduce_partials(C.part0, C.nparts_op);
+    const bool bad = !(pq > 0.0) || !isfinite(pq);
+    if (lead) S->done_r = bad ? 3 : 0;
+    if (bad) return false;
     a = S->rz2[S->iter & 1] / pq;
     return true;
 }
 
 // x += alpha p ; r -= alpha q ; partials r.r
 __global__ __launch_bounds__(256) void k_pcg_update(CGArgs C) {
-    if (C.S->done) return;
     double a, rr = 0.0;
     if (!pcg_alpha(C, a)) return;
     for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < C.n; i += int64_t(gridDim.x) * 256) {
@@ -1398,7 +1402,6 @@ __global__ __launch_bounds__(256) void k_pcg_update(CGArgs C) {
 // the lattice solver's update: x, r, the partials of r.r, and the start of the
 // FP32 pre-smoothing (b = r, x = D^-1 b / theta)
 __global__ __launch_bounds__(256) void k_pcg_update_lat(CGArgs C, MGLevelArgs L) {
-    if (C.S->done) return;
     double a, rr = 0.0;
     if (!pcg_alpha(C, a)) return;
     const float ith = float(L.cheb[0]);
@@ -1419,15 +1422,19 @@ __global__ __launch_bounds__(256) void k_pcg_update_lat(CGArgs C, MGLevelArgs L)
 template <typename T>
 __global__ __launch_bounds__(256) void k_pcg_p(CGArgs C, const T* __restrict__ z, int n, int first) {
     CGScalars* S = C.S;
-    if (S->done) return;
-    const double rz = reduce_partials(C.part0, n);
-    const int it = S->iter;
-    if (!(rz > 0.0) || !isfinite(rz)) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) S->done = 3;
+    const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
+    const int was = S->done_z;
+    if (was) {
+        if (lead) S->done = was;
         return;
     }
+    const double rz = reduce_partials(C.part0, n);
+    const int it = S->iter;
+    const bool bad = !(rz > 0.0) || !isfinite(rz);
+    if (lead) S->done = bad ? 3 : 0;
+    if (bad) return;
     const double beta = first ? 0.0 : rz / S->rz2[(it + 1) & 1];
-    if (blockIdx.x == 0 && threadIdx.x == 0) S->rz2[it & 1] = rz;
+    if (lead) S->rz2[it & 1] = rz;
     for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < C.n; i += int64_t(gridDim.x) * 256)
         C.p[i] = first ? double(z[i]) : double(z[i]) + beta * C.p[i];
 }
@@ -1435,7 +1442,7 @@ __global__ __launch_bounds__(256) void k_pcg_p(CGArgs C, const T* __restrict__ z
 // z = x0 + dlast (the level-0 V-cycle output) ; partials r.z
 __global__ __launch_bounds__(256) void k_pcg_rz(CGArgs C, const double* __restrict__ x0,
                                                 const double* __restrict__ dlast) {
-    if (C.S->done) return;
+    if (C.S->done_z) return;
     double rz = 0.0;
     for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < C.n; i += int64_t(gridDim.x) * 256) {
         const double z = dlast ? x0[i] + dlast[i] : x0[i];
@@ -1449,7 +1456,7 @@ __global__ __launch_bounds__(256) void k_pcg_rz(CGArgs C, const double* __restri
 __global__ __launch_bounds__(256) void k_pcg_rz_rank(CGArgs C, int nav, const int32_t* __restrict__ rank_of_lat,
                                                      const double* __restrict__ x0,
                                                      const double* __restrict__ dlast) {
-    if (C.S->done) return;
+    if (C.S->done_z) return;
     double rz = 0.0;
     for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < C.n; i += int64_t(gridDim.x) * 256) {
         const int64_t p = i / nav, k = int64_t(rank_of_lat[p]) * nav + (i - p * nav);
@@ -1484,7 +1491,7 @@ __global__ __launch_bounds__(256) void k_pcg_start_scalars(CGArgs C, double tol2
         S->iter = 0;
         S->tol2 = tol2;
         S->max_it = max_it;
-        S->done = (bb == 0.0) ? 1 : (isfinite(bb) ? 0 : 4);
+        S->done = S->done_z = (bb == 0.0) ? 1 : (isfinite(bb) ? 0 : 4);
     }
 }
 
@@ -1494,10 +1501,7 @@ __global__ __launch_bounds__(256) void k_pcg_recheck(CGArgs C) {
     if (threadIdx.x == 0) {
         CGScalars* S = C.S;
         S->rr = rr;
-        if (!isfinite(rr)) S->done = 4;
-        else if (rr <= S->tol2 * S->bb) S->done = 1;
-        else if (S->iter >= S->max_it) S->done = 2;
-        else S->done = 0;
+        S->done = S->done_z = !isfinite(rr) ? 4 : rr <= S->tol2 * S->bb ? 1 : S->iter >= S->max_it ? 2 : 0;
     }
 }
 
