@@ -91,3 +91,19 @@ def test_the_convergence_test_comes_before_the_vcycle_flag(name):
     body = _functions()[name][1]
     assert "*done" not in body
     assert body.index("pcg_check_block") < body.index("vcycle_done")
+
+
+def test_arguments_are_taken_after_the_hierarchy_is_built():
+    """mg_build may allocate anew what the solvers' arguments point to (the
+    partial sums of a large lattice): a function that calls it takes the arguments
+    after that."""
+    text = re.sub(r"//[^\n]*", "", open(os.path.join(CSRC, "context.hip")).read())
+    # functions at file level: their bodies' brace stands in column 0
+    bodies = re.findall(r"^\w[^\n;=]*\b(\w+)\(([^;{}]*)\)\s*\{\n(.*?)^\}", text, re.S | re.M)
+    seen = 0
+    for name, _, body in bodies:
+        if "mg_build(c)" in body:
+            seen += 1
+            args = re.search(r"\b(?:cg|bicg)_args\(c", body)
+            assert not args or body.rindex("mg_build(c)") < args.start(), name
+    assert seen >= 5
