@@ -16,6 +16,16 @@ __host__ __device__ constexpr int64_t xcd_block(int64_t b, int64_t nb) {
     return (b & 7) * (nb >> 3) + ((b & 7) < (nb & 7) ? (b & 7) : (nb & 7)) + (b >> 3);
 }
 
+// LDS written by a wave's lanes before this is seen by all of its lanes after
+// it, and what they read before is read: an exchange within the wave, for code
+// that the work-group's other waves do not pass through (no barrier; no
+// instruction beyond the waits for the wave's own LDS accesses)
+__device__ __forceinline__ void wave_exchange() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // block-level FP64 sum into partials[blockIdx.x] (blockDim 256)
 __device__ __forceinline__ void block_sum_store(double v, double* partials, int slot) {
     __shared__ double red[4];

@@ -511,7 +511,7 @@ __device__ __forceinline__ void stencil_layer(const MGLevelArgs& L, const float*
         for (int t = 0; t < NT; t++)
             if (t * kStenNodes + lane < kStenRun)
                 xs[row][t * kStenNodes + lane] = __longlong_as_double((long long)(uint64_t(q[row][t][1]) << 32 | q[row][t][0]));
-    __syncthreads();
+    wave_exchange();   // (xs is this wave's own; the waves come here by different ways)
     double y0 = 0.0, y1 = 0.0, y2 = 0.0;
 #pragma unroll
     for (int row = 0; row < 3; row++) {
