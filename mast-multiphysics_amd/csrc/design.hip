@@ -336,14 +336,14 @@ __global__ __launch_bounds__(64 * kOcWaves) void k_oc_sweep(int64_t n, const dou
     for (int64_t e = e0; e < e1; e += 64) {
         w[lane] = {r * sqrt(fmax(0.0, -c) / v), fmax(rho_min, r - move), fmin(1.0, r + move), v};
         if (e + 64 < e1) load(e + 64 + lane, r, c, v);
-        __builtin_amdgcn_wave_barrier();      // (LDS within a wave is in order)
+        wave_exchange();
         const int m = int(min(int64_t(64), e1 - e));
 #pragma unroll 8
         for (int j = 0; j < m; j++) {
             const double4 q = w[j];
             s = fma(q.w, oc_clamp(q.x, q.y, q.z, lam), s);
         }
-        __builtin_amdgcn_wave_barrier();
+        wave_exchange();                      // the batch is read; the next overwrites it
     }
     red[wave][lane] = s;
     __syncthreads();

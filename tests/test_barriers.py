@@ -26,3 +26,14 @@ def test_no_work_group_barrier_in_a_branch_on_the_wave():
     text = _text("mg_kernels.hip")
     assert re.search(r"if \(layer == 0\) stencil_layer<0>", text)
     assert "__syncthreads" not in _body(text, "stencil_layer")
+
+
+def test_exchanges_within_a_wave_are_fenced():
+    for f in sorted(os.listdir(CSRC)):
+        text = _text(f)
+        if f == "device_util.h":
+            body = _body(text, "wave_exchange")
+            assert body.count("__builtin_amdgcn_fence") == 2
+            assert body.index("__ATOMIC_RELEASE") < body.index("wave_barrier") < body.index("__ATOMIC_ACQUIRE")
+            text = text.replace(body, "")
+        assert "__builtin_amdgcn_wave_barrier" not in text, f
