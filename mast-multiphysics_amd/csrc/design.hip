@@ -128,7 +128,7 @@ int upload(mastg_design* d, Buf& b, const std::vector<T>& v) {
 
 // row e of the filter against the patterns seen so far: its number in id, a
 // new pattern when there is none; false once there are too many.  Weights
-// within tol (the rounding of the centroids' differences) are the same.
+// within tol are the same.
 bool row_pattern(int64_t e, const std::vector<std::pair<int32_t, double>>& row, double tol,
                  std::unordered_map<uint64_t, std::vector<int32_t>>& known, std::vector<int32_t>& ptr,
                  std::vector<FilterBatch>& pat, int32_t& id) {
@@ -476,10 +476,12 @@ int mastg_design_create(const mastg_problem_desc* desc, double radius, mastg_des
     std::vector<double> a, inv_s(n);
     std::vector<std::pair<int32_t, double>> row;
     // distinct rows: the same column offsets, the same weights to the rounding
-    // that the centroids' coordinates carry into their distances
+    // that the centroids' coordinates carry into their distances, but to 2^-40 of
+    // the radius wherever the mesh lies: far from the origin that rounding is as
+    // large as a mesh's own differences, and its rows stay their own
     double cmax = 0.0;
     for (const double x : c) cmax = std::max(cmax, std::fabs(x));
-    const double tol = 16.0 * 2.220446049250313e-16 * cmax;
+    const double tol = std::min(16.0 * 2.220446049250313e-16 * cmax, std::ldexp(radius, -40));
     std::unordered_map<uint64_t, std::vector<int32_t>> known;
     std::vector<int32_t> pat_id(size_t(n), 0), pat_ptr(1, 0);
     std::vector<FilterBatch> pat;
