@@ -241,8 +241,8 @@ __global__ __launch_bounds__(256) void k_filter(int64_t n, const int64_t* __rest
 // two waves of three mix patterns and read the entries per lane, 22 and 34 us.
 // Bound by the gathers (a 512-byte run per neighbour and wave): the
 // entries come in batches (three wide scalar loads, then kPatBatch gathers in
-// flight), a pattern padded
-// to whole batches with weights 0 on its own row.
+// flight), a pattern padded to whole batches with weights 0 on its own row, whose
+// products are left out (0 times an infinity there would be no number).
 __global__ __launch_bounds__(256) void k_filter_pattern(int n_waves, const int32_t* __restrict__ rows,
                                                         const int2* __restrict__ wave_pat,
                                                         const FilterBatch* __restrict__ pat,
@@ -265,7 +265,7 @@ __global__ __launch_bounds__(256) void k_filter_pattern(int n_waves, const int32
                 u[j] = (inv_s + P.off[j])[row];
             }
 #pragma unroll
-            for (int j = 0; j < kPatBatch; j++) s = fma(P.a[j], t[j] * u[j], s);
+            for (int j = 0; j < kPatBatch; j++) s = fma(P.a[j], P.a[j] != 0.0 ? t[j] * u[j] : 0.0, s);
         }
         out[row] = s;
     } else {
@@ -275,7 +275,7 @@ __global__ __launch_bounds__(256) void k_filter_pattern(int n_waves, const int32
 #pragma unroll
             for (int j = 0; j < kPatBatch; j++) t[j] = (in + P.off[j])[row];
 #pragma unroll
-            for (int j = 0; j < kPatBatch; j++) s = fma(P.a[j], t[j], s);
+            for (int j = 0; j < kPatBatch; j++) s = fma(P.a[j], P.a[j] != 0.0 ? t[j] : 0.0, s);
         }
         out[row] = s * inv_s[row];
     }

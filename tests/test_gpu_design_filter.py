@@ -47,3 +47,27 @@ def test_rows_that_nearly_agree(mastg, origin):
         y = M @ x
         assert np.max(np.abs(Dg.filter(x, transpose=t) - y)) <= 1e-12 * np.abs(y).max()
     Dg.close()
+
+
+# rows of 1 (padded by 15 to a batch), 16 (none), 17 and up to 27 neighbours
+@pytest.mark.parametrize("mesh,r", [((9, 1, 1), 0.5), ((16, 1, 1), 20.0), ((17, 1, 1), 20.0), ((9, 8, 7), 1.8)])
+def test_infinities_stay_where_they_belong(mastg, mesh, r):
+    """An infinite input makes the rows that hold it infinite, of its sign, and no
+    others; NaN likewise: as a sum over the row's neighbours gives it."""
+    print(f"[filter, infinities] {mesh} r = {r}", flush=True)
+    xyz, conn = _box(mesh)
+    Dg = _filter(mastg, xyz, conn, r)
+    W = D.filter_matrix(D.centroids(xyz, conn), r)
+    rng = np.random.default_rng(3)
+    n = len(conn)
+    for bad in (np.inf, -np.inf, np.nan):
+        x = rng.uniform(0.1, 1.0, n)
+        x[n // 2] = bad
+        for t, M in ((False, W), (True, W.T)):
+            y = np.array([sum(M[e, f] * x[f] for f in np.nonzero(M[e])[0]) for e in range(n)])
+            z = Dg.filter(x, transpose=t)
+            assert np.array_equal(np.isnan(z), np.isnan(y)) and np.array_equal(np.isinf(z), np.isinf(y))
+            assert np.array_equal(z[np.isinf(y)], y[np.isinf(y)])
+            ok = np.isfinite(y)
+            assert not ok.any() or np.max(np.abs(z[ok] - y[ok])) <= 1e-13 * np.abs(y[ok]).max()
+    Dg.close()
