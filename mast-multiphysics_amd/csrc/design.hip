@@ -55,7 +55,6 @@ constexpr double kOcLo = 1e-30, kOcHi = 1e30;   // the first bracket
 constexpr int kMaxPatterns = 4096;
 constexpr int kPatBatch = 16;
 constexpr int64_t kMaxPatternEntries = int64_t(1) << 19;
-constexpr int64_t kChipWaves = 8192;   // waves the chip holds at once (256 CUs, 8 per SIMD)
 
 // neighbours of a filter row: weights, and columns less the row's
 struct alignas(64) FilterBatch {
@@ -161,6 +160,35 @@ bool row_pattern(int64_t e, const std::vector<std::pair<int32_t, double>>& row, 
     }
     ptr.push_back(int32_t(pat.size()));
     return true;
+}
+
+// Whether the filter by patterns takes less time than by its CSR of nnz entries,
+// in units of 10 ps (both directions together).  The CSR streams its entries:
+// 0.58 each.  By patterns a wave's gather of one neighbour costs 8, or about one
+// for each line of memory its 64 rows lie in beyond 10 (rows that a mesh graded
+// along x scatters; ordinary ones lie in 5 to 20), whether its lanes hold rows or
+// padding, and a row's batches wait for each other: 2.5 us a batch of the longest
+// pattern.  Both forms measured (by patterns / CSR, us, there and back together):
+// 16^3 cells with 67 neighbours a row 27 / 13, each row its own pattern 47 / 14;
+// 32^3 35 / 23, 40^3 29 / 36, 48^3 44 / 61, 96x48x48 53 / 108, the same graded
+// along x 230 / 109, along z 50 / 109; with 19 neighbours 32^3 15 / 12, 40^3
+// 14 / 14, 48^3 16 / 20, 96x48x48 21 / 40; 5x200x200 with 65 neighbours 46 / 89.
+bool patterns_pay(const std::vector<int32_t>& pat_rows, const std::vector<int2>& wave_pat, int64_t nnz) {
+    int64_t cost = 0, longest = 0;
+    for (size_t w = 0; w < wave_pat.size(); w++) {
+        int64_t lines = 0, last = -1;
+        for (size_t l = 0; l < 64; l++) {
+            const int32_t r = pat_rows[w * 64 + l];   // ascending; -1 past the last
+            if (r >= 0 && r / 16 != last) {
+                lines++;
+                last = r / 16;
+            }
+        }
+        const int64_t batches = wave_pat[w].y - wave_pat[w].x;
+        cost += batches * kPatBatch * std::max<int64_t>(8, lines - 10);
+        longest = std::max(longest, batches);
+    }
+    return double(cost + 250000 * longest) < 0.58 * double(nnz);
 }
 
 // element volume (hex8, 2x2x2 Gauss: exact for the trilinear map's Jacobian)
@@ -514,8 +542,8 @@ int mastg_design_create(const mastg_problem_desc* desc, double radius, mastg_des
         if (patterns) patterns = row_pattern(e, row, tol, known, pat_ptr, pat, pat_id[size_t(e)]);
     }
     d->nnz = rp[n];
-    // rows grouped by pattern, a wave of 64 at a time; kept unless the padding
-    // of many small groups would cost more than the CSR saves
+    // rows grouped by pattern, a wave of 64 at a time; kept where that is the
+    // faster form
     std::vector<int32_t> pat_rows;
     std::vector<int2> wave_pat;
     if (patterns) {
@@ -525,9 +553,9 @@ int mastg_design_create(const mastg_problem_desc* desc, double radius, mastg_des
             for (int64_t w = 0; w < (first[k] + 63) / 64; w++) wave_pat.push_back(make_int2(pat_ptr[k - 1], pat_ptr[k]));
             first[k] = int64_t(wave_pat.size()) * 64;
         }
-        patterns = int64_t(wave_pat.size()) <= std::max(kChipWaves, n / 32);
         pat_rows.assign(wave_pat.size() * 64, -1);
         for (int64_t e = 0; e < n; e++) pat_rows[size_t(first[size_t(pat_id[size_t(e)])]++)] = int32_t(e);
+        patterns = patterns_pay(pat_rows, wave_pat, d->nnz);
     }
     d->n_waves = patterns ? int(wave_pat.size()) : 0;
     {
