@@ -834,6 +834,11 @@ int mg_build(mastg_ctx* c) {
         return fail(c, MASTG_ERR_INVALID, "multigrid unavailable: " + H.why);
     }
     const int nl = int(H.levels.size());
+    {   // the levels one work-group holds
+        std::vector<MGTailLevel> tl(static_cast<size_t>(nl));
+        for (int l = 0; l < nl; l++) tl[l] = {H.levels[l].nx, H.levels[l].ny, H.levels[l].nz, int(H.levels[l].n_nodes)};
+        c->mg_tail = mg_tail_first(tl.data(), nl, c->S.nav);
+    }
     std::vector<std::unique_ptr<MGLevelDev>> lv;
     for (int l = 0; l < nl; l++) {
         const MGLevelHost& h = H.levels[l];
@@ -959,7 +964,8 @@ int mg_build(mastg_ctx* c) {
             const size_t nb2 = size_t(nav) * nav;
             TRY(dalloc(c, L->Kel, size_t(S.n_elems) * S.npe * S.npe * nb2 * sizeof(double)));
             TRY(dalloc(c, L->val, size_t(S.n_blocks) * nb2 * sizeof(double)));
-            TRY(dalloc(c, L->val32, size_t(S.n_blocks) * nb2 * sizeof(float)));
+            // (only where launches of their own smooth the level)
+            if (l < c->mg_tail && l + 1 < nl) TRY(dalloc(c, L->val32, size_t(S.n_blocks) * nb2 * sizeof(float)));
             TRY(dalloc(c, L->dinv, nv));
             TRY(dalloc(c, L->r, nv));
             a.con = L->con.as<uint8_t>();
@@ -985,18 +991,12 @@ int mg_build(mastg_ctx* c) {
         }
         lv.push_back(std::move(L));
     }
-    // the levels one work-group holds
-    {
-        std::vector<MGTailLevel> tl(static_cast<size_t>(nl));
-        for (int l = 0; l < nl; l++) tl[l] = {H.levels[l].nx, H.levels[l].ny, H.levels[l].nz, int(H.levels[l].n_nodes)};
-        c->mg_tail = mg_tail_first(tl.data(), nl, c->S.nav);
-        if (c->mg_tail < nl) {
-            HipLock l(g_hip_mu);
-            HIPC(c, mg_tail_prepare());
-        }
-        for (int l = c->mg_tail; l + 1 < nl; l++)
-            TRY(dalloc(c, lv[l]->tail, size_t(mg_tail_entries(H.levels[l].dim, c->S.nav, H.levels[l].n_nodes)) * sizeof(float)));
+    if (c->mg_tail < nl) {
+        HipLock l(g_hip_mu);
+        HIPC(c, mg_tail_prepare());
     }
+    for (int l = c->mg_tail; l + 1 < nl; l++)
+        TRY(dalloc(c, lv[l]->tail, size_t(mg_tail_entries(H.levels[l].dim, c->S.nav, H.levels[l].n_nodes)) * sizeof(float)));
     if (c->d.physics == MASTG_HEX8_HEAT && std::min(nl - 1, c->mg_tail) > 1) {
         // heat: the first coarse level (lattice order) smooths with a 27-point
         // stencil too when it is above the tail and not the coarsest
