@@ -1189,7 +1189,8 @@ int mg_setup(mastg_ctx* c) {
             else launch_mg_to_stencil(C.a, C.sten.as<float>(), s);
         }
     }
-    launch_mg_power(P, kMGPowerIters, kMGPowerSafety, s);
+    if (!launch_mg_power(P, kMGPowerIters, kMGPowerSafety, s))
+        return fail(c, MASTG_ERR_INVALID, "power iteration is for 3 or 5 variables per node");
     // hex8 cells of several shapes (assembled problem level): [lam/30, lam]
     // (33 iterations at 3 steps on the distorted 128x64x64 against 35 at the
     // lattice's 80; 20 and 45 the same as 30)

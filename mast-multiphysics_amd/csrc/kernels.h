@@ -471,7 +471,7 @@ void launch_mg_rowinfo_nb(int nav, int64_t n_nodes, const int64_t* blk_ptr, cons
 // estimates of lambda_max(D^-1 A) by power iteration on the FP64 node blocks of
 // the n levels of P (n_it steps from a fixed positive start vector), times
 // `safety`, into their *lam; w0, w1: work vectors of nav n_nodes; part:
-// mg_power_partials(n) doubles; nav 3 or 5
+// mg_power_partials(n) doubles; nav 3 or 5 (false for another: nothing is launched)
 constexpr int kMGMaxLevels = 16;
 struct MGPowerLevel {
     int64_t n_nodes;
@@ -488,7 +488,7 @@ struct MGPowerArgs {
     int first[kMGMaxLevels + 1];       // set by the launcher
 };
 int64_t mg_power_partials(int n_levels);
-void launch_mg_power(MGPowerArgs P, int n_it, double safety, hipStream_t s);
+bool launch_mg_power(MGPowerArgs P, int n_it, double safety, hipStream_t s);
 void launch_mg_restrict(const MGLevelArgs& F, const MGLevelArgs& C, const int* done, hipStream_t s);
 // (F planar: the fine vectors are F's FP32 state)
 void launch_mg_prolong(const MGLevelArgs& F, const MGLevelArgs& C, const double* dlast, const int* done,

@@ -1570,12 +1570,14 @@ void launch_mg_rowinfo_nb(int nav, int64_t n_nodes, const int64_t* blk_ptr, cons
 // all the level's partials)
 constexpr int kPowerBlocks = 1024;
 int64_t mg_power_partials(int n_levels) { return 2 * int64_t(n_levels) * kPowerBlocks; }
-void launch_mg_power(MGPowerArgs P, int n_it, double safety, hipStream_t s) {
-    if (P.n <= 0) return;
+bool launch_mg_power(MGPowerArgs P, int n_it, double safety, hipStream_t s) {
+    if (P.n <= 0) return true;
+    if (P.nav != 3 && P.nav != 5) return false;
     P.first[0] = 0;
     for (int l = 0; l < P.n; l++) P.first[l + 1] = P.first[l] + std::min(nb_grid(P.level[l].n_nodes), kPowerBlocks);
     for (int it = 0; it < n_it; it++) hipLaunchKernelGGL(k_mg_power, dim3(P.first[P.n]), dim3(256), 0, s, P, it);
     hipLaunchKernelGGL(k_mg_power_lam, dim3(P.n), dim3(256), 0, s, P, n_it - 1, safety);
+    return true;
 }
 static int64_t lattice_blocks(const LatticeOpArgs& l) {
     return (int64_t(l.nx + 1) * (l.ny + 1) * (l.nz + 1) + 255) / 256;
