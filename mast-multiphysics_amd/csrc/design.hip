@@ -125,42 +125,54 @@ int upload(mastg_design* d, Buf& b, const std::vector<T>& v) {
     return MASTG_OK;
 }
 
-// row e of the filter against the patterns seen so far: its number in id, a
-// new pattern when there is none; false once there are too many.  Weights
-// within tol are the same.
-bool row_pattern(int64_t e, const std::vector<std::pair<int32_t, double>>& row, double tol,
-                 std::unordered_map<uint64_t, std::vector<int32_t>>& known, std::vector<int32_t>& ptr,
-                 std::vector<FilterBatch>& pat, int32_t& id) {
-    uint64_t h = 1469598103934665603ull;   // FNV-1a over the column offsets
-    for (const auto& p : row) h = (h ^ uint64_t(uint32_t(int32_t(p.first - e)))) * 1099511628211ull;
-    const size_t m = row.size(), nb = (m + kPatBatch - 1) / kPatBatch;
-    std::vector<int32_t>& same = known[h];
-    for (const int32_t k : same) {
-        const size_t b = size_t(ptr[size_t(k)]);
-        bool ok = size_t(ptr[size_t(k) + 1]) - b == nb;
-        for (size_t i = 0; i < m && ok; i++) {
+// Finds the rows that are copies of one another: the same column offsets, and
+// weights that agree to tol.
+struct RowPatterns {
+    double tol;
+    std::vector<int32_t> ptr{0};                 // pattern k: batches ptr[k] .. ptr[k + 1] of pat
+    std::vector<FilterBatch> pat;
+    std::unordered_map<uint64_t, std::vector<std::pair<double, int32_t>>> known;   // by their offsets' hash: weights' sum, number
+    int32_t last = -1;                           // the row before's
+
+    bool same(int32_t k, int64_t e, const int32_t* col, const double* a, size_t m) const {
+        const size_t b = size_t(ptr[size_t(k)]), nb = (m + kPatBatch - 1) / kPatBatch;
+        if (size_t(ptr[size_t(k) + 1]) - b != nb) return false;
+        for (size_t i = 0; i < m; i += kPatBatch) {
             const FilterBatch& P = pat[b + i / kPatBatch];
-            ok = P.off[i % kPatBatch] == int32_t(row[i].first - e) && std::fabs(P.a[i % kPatBatch] - row[i].second) <= tol;
+            const size_t q = std::min(m - i, size_t(kPatBatch));
+            bool ok = true;
+            for (size_t j = 0; j < q; j++)
+                ok &= (P.off[j] == int32_t(col[i + j] - e)) & (std::fabs(P.a[j] - a[i + j]) <= tol);
+            // (the rest of the last batch: this row is no shorter than the pattern)
+            for (size_t j = q; j < size_t(kPatBatch); j++) ok &= P.a[j] == 0.0;
+            if (!ok) return false;
         }
-        // (the rest of the last batch: this row is no shorter than the pattern)
-        for (size_t i = m; i < nb * kPatBatch && ok; i++) ok = pat[b + i / kPatBatch].a[i % kPatBatch] == 0.0;
-        if (ok) {
-            id = k;
-            return true;
+        return true;
+    }
+    // the number of row e's pattern (m columns and weights, their sum), a new one
+    // when there is none; -1 once there are too many
+    int32_t find(int64_t e, const int32_t* col, const double* a, size_t m, double sum) {
+        if (last >= 0 && same(last, e, col, a, m)) return last;
+        uint64_t h = m;                          // of the column offsets (no chain of products)
+        for (size_t i = 0; i < m; i++) h += uint64_t(int64_t(col[i] - e)) * (2 * i + 1);
+        std::vector<std::pair<double, int32_t>>& alike = known[h];
+        const double near = double(m) * (tol + 4.5e-16 * sum);   // sums of weights within tol, rounded m times
+        for (const auto& k : alike)
+            if (std::fabs(k.first - sum) <= near && same(k.second, e, col, a, m)) return last = k.second;
+        const size_t nb = (m + kPatBatch - 1) / kPatBatch;
+        if (int64_t(ptr.size()) > kMaxPatterns || int64_t(pat.size() + nb) * kPatBatch > kMaxPatternEntries) return -1;
+        last = int32_t(ptr.size()) - 1;
+        alike.push_back({sum, last});
+        pat.resize(pat.size() + nb, FilterBatch{});
+        for (size_t i = 0; i < m; i++) {
+            FilterBatch& P = pat[size_t(ptr[size_t(last)]) + i / kPatBatch];
+            P.a[i % kPatBatch] = a[i];
+            P.off[i % kPatBatch] = int32_t(col[i] - e);
         }
+        ptr.push_back(int32_t(pat.size()));
+        return last;
     }
-    if (int64_t(ptr.size()) > kMaxPatterns || int64_t(pat.size() + nb) * kPatBatch > kMaxPatternEntries) return false;
-    id = int32_t(ptr.size()) - 1;
-    same.push_back(id);
-    pat.resize(pat.size() + nb, FilterBatch{});
-    for (size_t i = 0; i < m; i++) {
-        FilterBatch& P = pat[size_t(ptr[size_t(id)]) + i / kPatBatch];
-        P.a[i % kPatBatch] = row[i].second;
-        P.off[i % kPatBatch] = int32_t(row[i].first - e);
-    }
-    ptr.push_back(int32_t(pat.size()));
-    return true;
-}
+};
 
 // Whether the filter by patterns takes less time than by its CSR of nnz entries,
 // in units of 10 ps (both directions together).  The CSR streams its entries:
@@ -173,22 +185,17 @@ bool row_pattern(int64_t e, const std::vector<std::pair<int32_t, double>>& row, 
 // 32^3 35 / 23, 40^3 29 / 36, 48^3 44 / 61, 96x48x48 53 / 108, the same graded
 // along x 230 / 109, along z 50 / 109; with 19 neighbours 32^3 15 / 12, 40^3
 // 14 / 14, 48^3 16 / 20, 96x48x48 21 / 40; 5x200x200 with 65 neighbours 46 / 89.
-bool patterns_pay(const std::vector<int32_t>& pat_rows, const std::vector<int2>& wave_pat, int64_t nnz) {
-    int64_t cost = 0, longest = 0;
-    for (size_t w = 0; w < wave_pat.size(); w++) {
-        int64_t lines = 0, last = -1;
-        for (size_t l = 0; l < 64; l++) {
-            const int32_t r = pat_rows[w * 64 + l];   // ascending; -1 past the last
-            if (r >= 0 && r / 16 != last) {
-                lines++;
-                last = r / 16;
-            }
+int64_t pattern_budget(int64_t nnz, int64_t longest_row) {   // what the waves' gathers may cost
+    return int64_t(0.58 * double(nnz)) - 250000 * ((longest_row + kPatBatch - 1) / kPatBatch);
+}
+int64_t pattern_wave_cost(int64_t batches, const int32_t* rows) {   // 64 rows, ascending, -1 past the last
+    int64_t lines = 0, last = -1;
+    for (int l = 0; l < 64; l++)
+        if (rows[l] >= 0 && rows[l] / 16 != last) {
+            lines++;
+            last = rows[l] / 16;
         }
-        const int64_t batches = wave_pat[w].y - wave_pat[w].x;
-        cost += batches * kPatBatch * std::max<int64_t>(8, lines - 10);
-        longest = std::max(longest, batches);
-    }
-    return double(cost + 250000 * longest) < 0.58 * double(nnz);
+    return batches * kPatBatch * std::max<int64_t>(8, lines - 10);
 }
 
 // element volume (hex8, 2x2x2 Gauss: exact for the trilinear map's Jacobian)
@@ -503,17 +510,14 @@ int mastg_design_create(const mastg_problem_desc* desc, double radius, mastg_des
     std::vector<int32_t> col;
     std::vector<double> a, inv_s(n);
     std::vector<std::pair<int32_t, double>> row;
-    // distinct rows: the same column offsets, the same weights to the rounding
+    // rows are copies of one another when their weights agree to the rounding
     // that the centroids' coordinates carry into their distances, but to 2^-40 of
     // the radius wherever the mesh lies: far from the origin that rounding is as
     // large as a mesh's own differences, and its rows stay their own
     double cmax = 0.0;
     for (const double x : c) cmax = std::max(cmax, std::fabs(x));
     const double tol = std::min(16.0 * 2.220446049250313e-16 * cmax, std::ldexp(radius, -40));
-    std::unordered_map<uint64_t, std::vector<int32_t>> known;
-    std::vector<int32_t> pat_id(size_t(n), 0), pat_ptr(1, 0);
-    std::vector<FilterBatch> pat;
-    bool patterns = true;
+    int64_t longest = 0;
     for (int64_t e = 0; e < n; e++) {
         row.clear();
         const int64_t ki = key(e, 0), kj = key(e, 1), kk = key(e, 2);
@@ -539,11 +543,24 @@ int mastg_design_create(const mastg_problem_desc* desc, double radius, mastg_des
         }
         inv_s[e] = 1.0 / s;
         rp[e + 1] = int64_t(col.size());
-        if (patterns) patterns = row_pattern(e, row, tol, known, pat_ptr, pat, pat_id[size_t(e)]);
+        longest = std::max(longest, int64_t(row.size()));
     }
     d->nnz = rp[n];
-    // rows grouped by pattern, a wave of 64 at a time; kept where that is the
-    // faster form
+    // the rows' patterns, looked for while they can be the faster form (a
+    // pattern fills a wave at least, at the least cost of its gathers)
+    int64_t budget = pattern_budget(d->nnz, longest), least = 0;
+    bool patterns = budget > 0;
+    RowPatterns rows{tol};
+    std::vector<int32_t> pat_id(patterns ? size_t(n) : 0);
+    const std::vector<int32_t>& pat_ptr = rows.ptr;
+    for (int64_t e = 0; e < n && patterns; e++) {
+        const size_t seen = rows.pat.size();
+        pat_id[size_t(e)] = rows.find(e, &col[size_t(rp[e])], &a[size_t(rp[e])], size_t(rp[e + 1] - rp[e]),
+                                     1.0 / inv_s[size_t(e)]);
+        least += int64_t(rows.pat.size() - seen) * kPatBatch * 8;
+        patterns = pat_id[size_t(e)] >= 0 && least < budget;
+    }
+    // grouped by pattern, a wave of 64 at a time; kept where that is the faster form
     std::vector<int32_t> pat_rows;
     std::vector<int2> wave_pat;
     if (patterns) {
@@ -555,7 +572,9 @@ int mastg_design_create(const mastg_problem_desc* desc, double radius, mastg_des
         }
         pat_rows.assign(wave_pat.size() * 64, -1);
         for (int64_t e = 0; e < n; e++) pat_rows[size_t(first[size_t(pat_id[size_t(e)])]++)] = int32_t(e);
-        patterns = patterns_pay(pat_rows, wave_pat, d->nnz);
+        for (size_t w = 0; w < wave_pat.size(); w++)
+            budget -= pattern_wave_cost(wave_pat[w].y - wave_pat[w].x, &pat_rows[w * 64]);
+        patterns = budget > 0;
     }
     d->n_waves = patterns ? int(wave_pat.size()) : 0;
     {
@@ -569,7 +588,7 @@ int mastg_design_create(const mastg_problem_desc* desc, double radius, mastg_des
     int rc;
     if (patterns)
         (rc = upload(d, d->pat_rows, pat_rows)) || (rc = upload(d, d->wave_pat, wave_pat)) ||
-            (rc = upload(d, d->pat, pat));
+            (rc = upload(d, d->pat, rows.pat));
     else
         (rc = upload(d, d->row_ptr, rp)) || (rc = upload(d, d->col, col)) || (rc = upload(d, d->a, a));
     if (rc || (rc = upload(d, d->inv_s, inv_s)) || (rc = upload(d, d->vol, vol)) ||
