@@ -594,14 +594,12 @@ int solve_stats(mastg_ctx* c, const double* r, const double* b, hipEvent_t e0, h
 int cg_loop(mastg_ctx* c, const CGArgs& a, const double* b, const mastg_solve_opts* o, int op, int chunk,
             hipEvent_t e0, hipEvent_t e1, mastg_solve_stats* st);
 
-// op: 0 FP64 CSR SpMV, 1 matrix-free FP64, 2 mixed precision (FP32 node-block
-// SpMV inside CG whose residual is replaced by the FP64 true residual b - A x
-// each time it has dropped by reliable_delta, and at convergence)
 // The lattice of the mesh for matrix-free CG, looked for on the first such solve
 // (any cell counts, unlike the multigrid hierarchy's).  On equal boxes the
 // lattice operator makes the product in one launch, without the element forces
 // that the general form writes and gathers: 46x24x24 nodes 5.1 us against
-// 9.5 + 7.1; an iteration there 23.4 -> 12.7 us.
+// 9.5 + 7.1; an iteration there 23.4 -> 12.7 us.  Its tables take 65 bytes per
+// node; where they find no room the general form solves.
 int mf_lattice(mastg_ctx* c) {
     MFLattice& M = c->mf_lat;
     if (M.tried) return MASTG_OK;
@@ -621,18 +619,34 @@ int mf_lattice(mastg_ctx* c) {
     for (int64_t p = 0; p < h.n_nodes; p++)
         for (int v = 0; v < 3; v++)
             if (c->S.constrained[size_t(h.rank_of_lat[p]) * 3 + v]) con[p] |= uint8_t(1 << v);
-    TRY(upload(c, M.rank_of_lat, h.rank_of_lat));
-    TRY(upload(c, M.elem_of_cell, h.elem_of_cell));
-    TRY(upload(c, M.nodecon, con));
-    TRY(dalloc(c, M.sE_cell, size_t(h.n_elems) * sizeof(double)));
-    TRY(dalloc(c, M.dinv, size_t(c->S.n_active) * sizeof(double)));
-    TRY(dalloc(c, M.b, size_t(c->S.n_active) * sizeof(double)));
+    auto tables = [&]() -> int {
+        TRY(upload(c, M.rank_of_lat, h.rank_of_lat));
+        TRY(upload(c, M.elem_of_cell, h.elem_of_cell));
+        TRY(upload(c, M.nodecon, con));
+        TRY(dalloc(c, M.sE_cell, size_t(h.n_elems) * sizeof(double)));
+        TRY(dalloc(c, M.dinv, size_t(c->S.n_active) * sizeof(double)));
+        return dalloc(c, M.b, size_t(c->S.n_active) * sizeof(double));
+    };
+    const int rc = tables();
+    if (rc == MASTG_ERR_OOM) {
+        (void)hipGetLastError();
+        c->err.clear();
+        for (DevBuf* b : {&M.rank_of_lat, &M.elem_of_cell, &M.nodecon, &M.sE_cell, &M.dinv, &M.b}) {
+            c->device_bytes -= int64_t(b->bytes);
+            b->release();
+        }
+        return MASTG_OK;
+    }
+    TRY(rc);
     M.op.sE_cell = M.sE_cell.as<double>();
     M.op.nodecon = M.nodecon.as<uint8_t>();
     M.ok = true;
     return MASTG_OK;
 }
 
+// op: 0 FP64 CSR SpMV, 1 matrix-free FP64, 2 mixed precision (FP32 node-block
+// SpMV inside CG whose residual is replaced by the FP64 true residual b - A x
+// each time it has dropped by reliable_delta, and at convergence)
 int cg_solve(mastg_ctx* c, const double* b, const mastg_solve_opts* o, mastg_solve_stats* st, int op) {
     const bool matfree = op == 1;
     const Structure& S = c->S;
