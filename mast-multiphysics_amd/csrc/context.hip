@@ -613,7 +613,8 @@ int mf_lattice(mastg_ctx* c) {
     }
     M.op.nx = h.nx; M.op.ny = h.ny; M.op.nz = h.nz;
     M.op.is_box = 1;
-    if (!box_operator(Kh.data(), M.op.box) || lattice_partials(M.op) > int64_t(c->part0.bytes / sizeof(double)))
+    if (!box_operator(Kh.data(), M.op.box) || !box_apply_pays(M.op) ||
+        lattice_partials(M.op) > int64_t(c->part0.bytes / sizeof(double)))
         return MASTG_OK;
     std::vector<uint8_t> con(static_cast<size_t>(h.n_nodes), 0);
     for (int64_t p = 0; p < h.n_nodes; p++)

@@ -456,6 +456,7 @@ void launch_lattice_apply(const CGArgs& c, const double* x, double* y, hipStream
 // the same two on a lattice of axis-aligned boxes (l.is_box; lattice_box.hip)
 int64_t box_partials(const LatticeOpArgs& l);
 int64_t box_partials_most(const LatticeOpArgs& l);
+bool box_apply_pays(const LatticeOpArgs& l);   // matrix-free CG's product is faster by it
 void launch_box_apply(const LatticeOpArgs& l, const double* x, double* y, double* part, const int* done, hipStream_t s);
 void launch_box_smooth(const LatticeOpArgs& l, const LatSmooth& S, const int* done, hipStream_t s);
 // inverse diagonal of the lattice operator (component-major lattice order,

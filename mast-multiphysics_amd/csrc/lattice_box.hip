@@ -355,6 +355,17 @@ bool box_operator(const double* Khat, BoxOp<double>& op) {
     return big > 0.0;
 }
 
+// Against the element-wise product of matrix-free CG: a plane of a few points
+// fills little of its wave, and each wave costs the same.  An iteration takes
+// about 10.5 us + 1.4 ns a wave + 0.045 ns a point here and 20.4 us + 0.1 ns a
+// point there; measured (here / there, us): 1x1x8000 cells 21 / 23, 1x1x12000
+// 27 / 25, 1x1x40000 70 / 35, 2x2x12000 31 / 35, 2x2x30000 62 / 46, 3x3x16000
+// 44 / 49, 5x5x8000 37 / 59, 45x23x23 12.7 / 23.4.
+bool box_apply_pays(const LatticeOpArgs& l) {
+    const int64_t points = int64_t(l.nx + 1) * (l.ny + 1) * (l.nz + 1);
+    return box_waves(l, 1) <= 7600 + points / 23;
+}
+
 int64_t box_partials_most(const LatticeOpArgs& l) { return box_blocks(l, 1); }
 int64_t box_partials(const LatticeOpArgs& l) { return box_blocks(l, box_layers(l)); }
 
