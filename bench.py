@@ -590,8 +590,10 @@ def main():
     if head == "mg":
         # dominant kernel: the FP32 smoothing step on the problem level (12
         # launches per V-cycle, one V-cycle per CG iteration); the FP64 CG
-        # product (one launch per iteration) beside it.  In the box's modes
-        # neither does much arithmetic: bytes are the bound
+        # product (one launch per iteration) beside it.  Both issue vector
+        # instructions longer than their bytes take (8.8 us of 12.7 against 7.2
+        # by the counters in profiles/), most of them not the operator's own
+        # arithmetic; rated by their bytes, which a better form could not avoid
         wl = f"hex8 {nx}x{ny}x{nz}"
         s_ms = ctx.bench_kernel(8, 20)
         k_ms = ctx.bench_kernel(6, 20)
@@ -605,7 +607,8 @@ def main():
                 "traffic": measured_traffic("k_box_smooth", wl), "avg_launch_ms": s_ms,
                 "algorithmic_flops": fl, "algorithmic_bytes": sbyt,
                 "flops_view_tflops": fl / (s_ms * 1e-3) / 1e12,
-                "note": "one round of waves: loads and arithmetic of a wave follow each other",
+                "note": ("one round of waves: VALU issue takes 8.8 us, the measured traffic 7.2 us at the copy "
+                         "rate, and they overlap only in part"),
                 "fp64_cg_operator": {
                     "kernel": "k_box_apply (FP64 lattice operator)", "avg_launch_ms": k_ms,
                     "achieved": a64, "peak": PEAK_HBM_GBS, "unit": "GB/s", "frac": a64 / PEAK_HBM_GBS,

@@ -56,10 +56,10 @@ def test_filter_and_volume(oracle, mastg, kind, mesh, r_h, distort):
     Dg.close()
 
 
-# rows by pattern: every row its own pattern (4 x 4 x 4, the ball covers the
-# mesh), one element, waves of 64 rows cut by every boundary, a pattern of
-# exactly one batch of 16 and of 17; and more distinct rows than patterns are
-# kept for (displaced nodes: the CSR)
+# meshes too small for the filter by row patterns, which has tests of its own
+# (test_gpu_design_filter.py): every row its own (4 x 4 x 4, the ball covers the
+# mesh), one element, rows cut by every boundary, of 16 and of 17 neighbours, and
+# displaced nodes
 @pytest.mark.parametrize("mesh,r_h,distort", [((4, 4, 4), 9.0, 0.0), ((1, 1, 1), 1.5, 0.0), ((65, 2, 3), 1.5, 0.0),
                                               ((64, 4, 4), 1.2, 0.0), ((16, 1, 1), 20.0, 0.0), ((17, 1, 1), 20.0, 0.0),
                                               ((20, 16, 16), 1.8, 0.2)])
